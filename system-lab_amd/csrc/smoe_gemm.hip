@@ -38,6 +38,7 @@
 // (no host sync, no workspace) and leaves when its tile index is past the
 // real total.  Zero-token experts own no tiles; rows past an expert's end are
 // clamped on load and masked on store.
+#include "smoe_gemm_small.h"
 #include "smoe_mfma.h"
 
 namespace smoe {
@@ -405,6 +406,9 @@ extern "C" int smoe_grouped_gemm_fp8(const uint8_t* a, const float* as, const ui
   SMOE_CHECK_PTR(c);
   if (!as || !bs || !offsets) return SMOE_EINVAL_NULL;
   if (((uintptr_t)as | (uintptr_t)bs | (uintptr_t)offsets) & 3u) return SMOE_EINVAL_PTRALIGN;
+  if (small_gemm_rows(SmallWeights::kPlain, E, R))
+    return small_gemm_launch(SmallWeights::kPlain, false, a, as, b, bs, offsets, E, R, N, Kdim, c,
+                             nullptr, nullptr, (hipStream_t)stream);
   using C = GemmCfg;
   const long long mt_bound = (R + C::kBM - 1) / C::kBM + E;
   const long long NT = (N + C::kBN - 1) / C::kBN;
@@ -441,8 +445,11 @@ extern "C" int smoe_grouped_gemm_fp8_swiglu(const uint8_t* a, const float* as, c
   if (!as || !w1s || !offsets || !hs) return SMOE_EINVAL_NULL;
   if (((uintptr_t)as | (uintptr_t)w1s | (uintptr_t)offsets | (uintptr_t)hs) & 3u)
     return SMOE_EINVAL_PTRALIGN;
-  using C = GemmCfg;
   const int N = 2 * I;
+  if (small_gemm_rows(SmallWeights::kPlain, E, R))
+    return small_gemm_launch(SmallWeights::kPlain, false, a, as, w1, w1s, offsets, E, R, N, Kdim,
+                             c1, hq, hs, (hipStream_t)stream);
+  using C = GemmCfg;
   const long long mt_bound = (R + C::kBM - 1) / C::kBM + E;
   const long long NT = I / kGroup;
   const long long mt_pad = (mt_bound + kChipM - 1) / kChipM * kChipM;

@@ -29,6 +29,7 @@
 //
 // Scope: K a multiple of 128 from 512 to 65536 (K blocks 4 .. 512), every
 // scale a power of two; the ops layer checks the recipe.
+#include "smoe_gemm_small.h"
 #include "smoe_mfma.h"
 
 namespace smoe {
@@ -443,6 +444,9 @@ extern "C" int smoe_grouped_gemm_fp8_packed_e8m0(const uint8_t* a, const float* 
   const int st = e8m0_args(a, as, wp, ws, offsets, E, R, N, Kdim);
   if (st) return st;
   SMOE_CHECK_PTR(c);
+  if (small_gemm_rows(SmallWeights::kPacked, E, R))
+    return small_gemm_launch(SmallWeights::kPacked, true, a, as, wp, ws, offsets, E, R, N, Kdim, c,
+                             nullptr, nullptr, (hipStream_t)stream);
   long long mt_bound;
   const long long nblk = e8m0_grid(E, R, (N + e8m0::kBN - 1) / e8m0::kBN, &mt_bound);
   if (nblk > 0x7fffffffLL) return SMOE_EINVAL_DIM;
@@ -465,6 +469,9 @@ extern "C" int smoe_grouped_gemm_fp8_packed_e8m0_swiglu(const uint8_t* a, const 
   if (c1 && ((uintptr_t)c1 & 15u)) return SMOE_EINVAL_PTRALIGN;
   if (!hs) return SMOE_EINVAL_NULL;
   if ((uintptr_t)hs & 3u) return SMOE_EINVAL_PTRALIGN;
+  if (small_gemm_rows(SmallWeights::kPacked, E, R))
+    return small_gemm_launch(SmallWeights::kPacked, true, a, as, w1p, w1s, offsets, E, R, 2 * I,
+                             Kdim, c1, hq, hs, (hipStream_t)stream);
   long long mt_bound;
   const long long nblk = e8m0_grid(E, R, I / kGroup, &mt_bound);
   if (nblk > 0x7fffffffLL) return SMOE_EINVAL_DIM;

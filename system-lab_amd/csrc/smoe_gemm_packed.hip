@@ -36,6 +36,7 @@
 //
 // Scope: K a multiple of 512 (the chunked activation scales); other K use the
 // plain kernel (the ops layer and SimpleMoE choose).
+#include "smoe_gemm_small.h"
 #include "smoe_mfma.h"
 
 namespace smoe {
@@ -426,6 +427,9 @@ extern "C" int smoe_grouped_gemm_fp8_packed(const uint8_t* a, const float* as, c
   const int st = packed_args(a, as, wp, ws, offsets, E, R, N, Kdim);
   if (st) return st;
   SMOE_CHECK_PTR(c);
+  if (small_gemm_rows(SmallWeights::kPacked, E, R))
+    return small_gemm_launch(SmallWeights::kPacked, false, a, as, wp, ws, offsets, E, R, N, Kdim,
+                             c, nullptr, nullptr, (hipStream_t)stream);
   long long mt_bound;
   const long long nblk = packed_grid(E, R, (N + packed::kBN - 1) / packed::kBN, &mt_bound);
   if (nblk > 0x7fffffffLL) return SMOE_EINVAL_DIM;
@@ -448,6 +452,9 @@ extern "C" int smoe_grouped_gemm_fp8_packed_swiglu(const uint8_t* a, const float
   if (c1 && ((uintptr_t)c1 & 15u)) return SMOE_EINVAL_PTRALIGN;
   if (!hs) return SMOE_EINVAL_NULL;
   if ((uintptr_t)hs & 3u) return SMOE_EINVAL_PTRALIGN;
+  if (small_gemm_rows(SmallWeights::kPacked, E, R))
+    return small_gemm_launch(SmallWeights::kPacked, false, a, as, w1p, w1s, offsets, E, R, 2 * I,
+                             Kdim, c1, hq, hs, (hipStream_t)stream);
   long long mt_bound;
   const long long nblk = packed_grid(E, R, I / kGroup, &mt_bound);
   if (nblk > 0x7fffffffLL) return SMOE_EINVAL_DIM;

@@ -1,0 +1,414 @@
+// smoe_gemm_small.hip — the dropless fp8 grouped GEMM for few rows per expert
+// (decode batches, short prompt chunks), for gfx950.
+//
+//   c[r,n] = bf16( sum_kb as[r,kb] * bs[e,n/128,kb] * sum_{k in kb} a[r,k]*b[e,n,k] )
+//
+// Contract, K orders and arithmetic per output are those of the 256-row
+// kernels (smoe_gemm.hip for plain weights, smoe_gemm_packed.hip for packed
+// ones, smoe_gemm_e8m0.hip for power-of-two scales), so the bytes are the
+// same.  What differs is the shape of the problem: with a few dozen rows per
+// expert every weight byte is used by one tile or two, and the time is that
+// of streaming the weights of the experts that have rows from HBM.
+//
+// Tiling.  A workgroup of 4 waves owns up to 96 rows x 64*kCB columns; wave w
+// owns all rows and columns w*16*kCB .. +16*kCB.  The weights go straight
+// from memory to the MFMA operand registers (nothing else in the workgroup
+// needs them), kD K steps ahead.  The row count of a tile picks its loop: 1,
+// 2, 4 or 6 blocks of 16 rows, so a tile of one row does a sixteenth of a
+// 256-row tile's MFMAs.  The activations of a tile pass through LDS in chunks
+// of at most 16 KiB (8, 4, 2 or 1 K steps), loaded to registers a chunk ahead
+// and written to the other half of the buffer at the chunk's end: one barrier
+// a chunk.  All loads are ordinary ones, so the compiler counts and waits for
+// each.  At most 256 registers and 51 KiB of LDS leave two workgroups per
+// CU, so one tile's start and end hide behind the other's stream.
+//
+// Every wave finds the workgroup's tile by itself (wave scans over the
+// experts' tile counts): no LDS and no barrier before the first load.
+// Tiles are numbered expert by expert and dealt to the XCDs in 8 contiguous
+// ranges; within an expert the row tiles of one column tile are neighbours,
+// so they share the weights in one L2 (with the column tiles fastest, 100
+// rows an expert at N = 28672, K = 4096 took 294 us against 237).
+//
+// Measured against the 256-row kernels (router loads, us before -> after):
+// H 4096, I 14336, E 8, 32 tokens top-2: fc1 with SwiGLU 261 -> 160 (5.9 TB/s
+// of weights), fc2 162 -> 81 (5.8 TB/s); H 2048, I 768, E 128, top-8: fc1 with
+// SwiGLU 29 -> 20 at 1 token, 122 -> 70 at 64 (5.8 TB/s), 125 -> 97 at 1000;
+// its fc2 on plain weights 65 -> 40 at 64 tokens, with E8M0 scales 72 -> 33.
+#include "smoe_gemm_small.h"
+#include "smoe_mfma.h"
+
+namespace smoe {
+namespace small {
+
+constexpr int kThreads = 256, kWaves = 4, kBM = 96;
+constexpr int kMaxChunk = 16 * 1024;  // most activation bytes of a chunk
+
+struct Tile {
+  int row0, rows, e, nt;
+};
+
+// The tile of workgroup bid: false when it is past the last one.  offsets[] is
+// device data the host never sees: whatever it holds, rows stay in [0, R).
+__device__ __forceinline__ bool find_tile(const int32_t* __restrict__ offsets, int E, int R, int NT,
+                                          int mt_bound, int bid, int lane, Tile& t) {
+  auto tiles = [&](int e) {
+    const int o0 = offsets[min(e, E)], o1 = offsets[min(e + 1, E)];
+    return o1 > o0 ? min((o1 - o0 + kBM - 1) / kBM, mt_bound) : 0;
+  };
+  auto scan = [&](int v) {
+#pragma unroll
+    for (int o = 1; o < kWave; o <<= 1) {
+      const int u = __shfl_up(v, o, kWave);
+      if (lane >= o) v += u;
+    }
+    return v;
+  };
+  constexpr int kHeld = 4;  // experts a lane keeps between the two passes
+  int cnt[kHeld], inc[kHeld];
+#pragma unroll
+  for (int i = 0; i < kHeld; ++i) cnt[i] = tiles(i * kWave + lane);
+  int total = 0;
+#pragma unroll
+  for (int i = 0; i < kHeld; ++i) {
+    if (i * kWave < E) {
+      inc[i] = scan(cnt[i]);
+      total = min(total + __builtin_amdgcn_readlane(inc[i], kWave - 1), mt_bound);
+    }
+  }
+  for (int b = kHeld * kWave; b < E; b += kWave) {
+    const int v = scan(tiles(b + lane));
+    total = min(total + __builtin_amdgcn_readlane(v, kWave - 1), mt_bound);
+  }
+  // 8 contiguous ranges of tiles, one per XCD; an expert's row tiles of one
+  // column tile are neighbours, so its weights are read from memory once
+  const int all = total * NT;
+  const int chunk = (all + 7) / 8;
+  const int j = bid >> 3, tl = (bid & 7) * chunk + j;
+  if (j >= chunk || tl >= all) return false;
+  const int mt = tl / NT;  // a row tile of the expert
+  int carry = 0, nt_e = 1, first = 0;
+  auto take = [&](int b, int c, int v) {  // the 64 experts from b: counts c, inclusive scan v
+    const uint64_t past = __ballot(carry + v > mt);
+    if (!past) {
+      carry += __builtin_amdgcn_readlane(v, kWave - 1);
+      return false;
+    }
+    const int l = __builtin_ctzll(past);
+    t.e = b + l;
+    nt_e = __builtin_amdgcn_readlane(c, l);
+    first = carry + __builtin_amdgcn_readlane(v, l) - nt_e;
+    return true;
+  };
+  bool found = false;
+#pragma unroll
+  for (int i = 0; i < kHeld; ++i)
+    if (!found && i * kWave < E) found = take(i * kWave, cnt[i], inc[i]);
+  for (int b = kHeld * kWave; b < E && !found; b += kWave) {
+    const int c = tiles(b + lane);
+    found = take(b, c, scan(c));
+  }
+  if (!found || t.e >= E) return false;
+  const int q = tl - first * NT;
+  t.nt = q / nt_e;
+  // the expert's n rows in nt_e = ceil(n / kBM) tiles of equal height, a
+  // multiple of 16: at most kBM, so the last one is never empty
+  const int o0 = offsets[t.e], o1 = offsets[t.e + 1];
+  const int h = min(((o1 - o0 + nt_e - 1) / nt_e + 15) & ~15, kBM);
+  t.row0 = o0 + (q - t.nt * nt_e) * h;
+  t.rows = min(h, min(o1, R) - t.row0);
+  return t.row0 >= 0 && t.rows > 0;
+}
+
+__device__ __forceinline__ int e8m0_of(float s) { return (__float_as_uint(s) >> 23) & 0xff; }
+
+__device__ __forceinline__ v8i lds_frag2(const uint8_t* base, int row, int c0, int c1) {
+  const v4i lo = *(const v4i*)(base + swz(row, c0));
+  const v4i hi = *(const v4i*)(base + swz(row, c1));
+  return __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
+}
+
+// The K loop of a tile of at most 16*kRB rows and its bf16 result staged in
+// LDS (row pitch kCPitch).  kD: K steps the weights are loaded ahead.
+template <SmallWeights kLay, bool kE8, int kCB, int kRB, int kD>
+__device__ __forceinline__ void run_tile(const uint8_t* __restrict__ a_base,
+                                         const float* __restrict__ s_base,
+                                         const uint8_t* __restrict__ b_base,
+                                         const float* __restrict__ sb_row, const uint32_t (&ob)[kCB],
+                                         int rows, int Kd, int ksb, uint8_t* smem, int tid) {
+  constexpr int kS = kRB <= 2 ? 8 / kRB : kRB == 4 ? 2 : 1;  // K steps per chunk
+  constexpr int kStep = kRB * 16 * kRow;  // LDS bytes per step
+  constexpr int kChunk = kS * kStep, kQ = kChunk / (kThreads * 16);
+  constexpr int kWords = kS * kRB * 16;  // activation scales of a chunk
+  constexpr bool kPacked = kLay == SmallWeights::kPacked;
+  constexpr int kHalf = kPacked ? 1024 : 16;     // a weight fragment's second 16 bytes
+  constexpr int kKStep = kPacked ? 2048 : kBK;   // weight bytes from one K block to the next
+  constexpr int kCPitch = 64 * kCB * 2 + 16;
+  static_assert(kQ * kThreads * 16 == kChunk && kChunk <= kMaxChunk && kWords <= kThreads, "chunk");
+  const int lane = tid & 63, wid = tid >> 6;
+  const int frow = lane & 15, fg = lane >> 4;
+
+  // this thread's 16-byte pieces of a chunk: 1 KiB segment q*4 + wid
+  // holds 8 row positions of one step (layout as in smoe_mfma.h)
+  uint32_t oa[kQ];
+  int sa[kQ];
+#pragma unroll
+  for (int q = 0; q < kQ; ++q) {
+    const int seg = q * kWaves + wid;
+    const int st = seg / (kRB * 2), rg = seg % (kRB * 2);
+    const int row = tile_row(rg * 8 + (lane >> 3));
+    oa[q] = (uint32_t)(min(row, rows - 1) * Kd + (((lane & 7) ^ (row & 7)) << 4));
+    sa[q] = st;
+  }
+  // threads below kWords also carry one activation scale
+  const int s_row = tid % (kRB * 16), s_st = (tid / (kRB * 16)) % kS;
+  const uint32_t os = (uint32_t)(min(s_row, rows - 1) * ksb);
+  v4i stg[kQ];
+  float sstg;
+  auto fetch = [&](int kc) {  // the chunk from K step kc (steps past the end repeat the last)
+#pragma unroll
+    for (int q = 0; q < kQ; ++q)
+      stg[q] = *(const v4i*)(a_base + oa[q] + (size_t)min(kc + sa[q], ksb - 1) * kBK);
+    sstg = s_base[os + min(kc + s_st, ksb - 1)];
+  };
+  auto stash = [&](int half) {
+    uint8_t* d = smem + half * kChunk + wid * 1024 + lane * 16;
+#pragma unroll
+    for (int q = 0; q < kQ; ++q) *(v4i*)(d + q * kWaves * 1024) = stg[q];
+    if (tid < kWords) ((float*)(smem + 2 * kChunk))[half * kWords + tid] = sstg;
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+  };
+
+  v8i w[kD][kCB];
+  auto load_w = [&](int kb, v8i (&f)[kCB]) {
+    const uint8_t* base = b_base + (size_t)kb * kKStep;
+#pragma unroll
+    for (int j = 0; j < kCB; ++j) {
+      const v4i lo = *(const v4i*)(base + ob[j]);
+      const v4i hi = *(const v4i*)(base + ob[j] + kHalf);
+      f[j] = __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
+    }
+  };
+  // activation fragment of 16 tile rows, lane group fg's share of the K block
+  // in the weights' order
+  auto frag = [&](const uint8_t* sA, int i) {
+    const int r = i * 16 + frow;
+    return kPacked ? lds_frag2(sA, r, fg, fg + 4) : lds_frag2(sA, r, fg * 2, fg * 2 + 1);
+  };
+  v4f acc[kRB][kCB];
+#pragma unroll
+  for (int i = 0; i < kRB; ++i)
+#pragma unroll
+    for (int j = 0; j < kCB; ++j) acc[i][j] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
+
+  fetch(0);
+#pragma unroll
+  for (int d = 0; d < kD; ++d) load_w(min(d, ksb - 1), w[d]);
+  // the weight scales of 64 K steps, lane l holding step l of them
+  float sbv = sb_row[min(lane, ksb - 1)], sbn = sb_row[min(64 + lane, ksb - 1)];
+  stash(0);
+
+  auto step = [&](int kb, v8i (&f)[kCB]) {
+    const int half = (kb / kS) & 1;
+    const uint8_t* sA = smem + half * kChunk + (kb % kS) * kStep;
+    const float* sS = (const float*)(smem + 2 * kChunk) + half * kWords + (kb % kS) * kRB * 16;
+    const float sb = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(sbv), kb & 63));
+    v8i fx = frag(sA, 0);
+#pragma unroll
+    for (int i = 0; i < kRB; ++i) {
+      v8i fxn = fx;
+      if (i + 1 < kRB) fxn = frag(sA, i + 1);
+      // the empty asm statements keep the row blocks in order (without them
+      // the compiler holds the results of a whole step at once)
+      asm volatile("" : "+v"(fx));
+      if constexpr (kE8) {
+        const int ew = e8m0_of(sb), ex = e8m0_of(sS[i * 16 + frow]);
+#pragma unroll
+        for (int j = 0; j < kCB; ++j)
+          acc[i][j] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(f[j], fx, acc[i][j], 0, 0, 0, ew, 0, ex);
+#pragma unroll
+        for (int j = 0; j < kCB; ++j) asm volatile("" : "+v"(acc[i][j]));
+      } else {
+        const float sc = sS[i * 16 + frow] * sb;
+        v4f p[kCB];
+#pragma unroll
+        for (int j = 0; j < kCB; ++j) p[j] = mfma16(f[j], fx, v4f{0.0f, 0.0f, 0.0f, 0.0f});
+#pragma unroll
+        for (int j = 0; j < kCB; ++j) {
+#pragma unroll
+          for (int v = 0; v < 4; ++v) acc[i][j][v] = __builtin_fmaf(p[j][v], sc, acc[i][j][v]);
+          asm volatile("" : "+v"(acc[i][j]));
+        }
+      }
+      fx = fxn;
+    }
+    // the buffer just used takes the weights kD steps ahead
+    load_w(min(kb + kD, ksb - 1), f);
+    asm volatile("" ::: "memory");
+  };
+  auto at = [&](int kb, v8i (&f)[kCB]) {
+    if (kb % kS == 0) fetch(kb + kS);
+    step(kb, f);
+    if (kb % kS == kS - 1) {
+      if ((kb & 63) == 63) {  // kS divides 64
+        sbv = sbn;
+        sbn = sb_row[min(kb + 65 + lane, ksb - 1)];
+      }
+      stash(((kb / kS) & 1) ^ 1);
+    }
+  };
+  int kb = 0;
+  for (; kb + kD <= ksb; kb += kD) {
+#pragma unroll
+    for (int d = 0; d < kD; ++d) at(kb + d, w[d]);
+  }
+#pragma unroll
+  for (int d = 0; d < kD - 1; ++d)
+    if (kb + d < ksb) at(kb + d, w[d]);
+
+  // ---- bf16 tile over the chunk buffers (every wave is done with them)
+  asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+#pragma unroll
+  for (int i = 0; i < kRB; ++i)
+#pragma unroll
+    for (int j = 0; j < kCB; ++j) {
+      uint2 o;
+      o.x = bf16_pack2(acc[i][j][0], acc[i][j][1]);
+      o.y = bf16_pack2(acc[i][j][2], acc[i][j][3]);
+      *(uint2*)(smem + (i * 16 + frow) * kCPitch + (wid * 16 * kCB + j * 16 + fg * 4) * 2) = o;
+    }
+}
+
+template <SmallWeights kLay, bool kE8, bool kSwiGLU, int kCB>
+__global__ __launch_bounds__(kThreads, 2) void gemm_small_kernel(
+    const uint8_t* __restrict__ a, const float* __restrict__ as, const uint8_t* __restrict__ b,
+    const float* __restrict__ bs, const int32_t* __restrict__ offsets, int E, int R, int N, int Kd,
+    int mt_bound, uint16_t* __restrict__ c, uint8_t* __restrict__ hq, float* __restrict__ hs) {
+  static_assert(!kSwiGLU || kCB == 4, "fused SwiGLU pairs 128 gate with 128 up columns");
+  constexpr int kBN = 64 * kCB, kCPitch = kBN * 2 + 16;
+  constexpr int kLoop = 2 * kMaxChunk + 2 * kThreads * 4;
+  constexpr int kSmem = kLoop > kBM * kCPitch ? kLoop : kBM * kCPitch;
+  __shared__ __attribute__((aligned(1024))) uint8_t smem[kSmem];
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wid = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int I = N / 2;
+  const int NT = kSwiGLU ? I / kGroup : (N + kBN - 1) / kBN;
+  Tile t;
+  if (!find_tile(offsets, E, R, NT, mt_bound, blockIdx.x, lane, t)) return;  // the whole workgroup leaves
+  const int e = t.e, row0 = t.row0, rows = t.rows, nt = t.nt;
+  const int n0 = nt * kBN, ksb = Kd / kBK, NB = (N + kGroup - 1) / kGroup;
+
+  const uint8_t* a_base = a + (size_t)row0 * Kd;
+  const float* s_base = as + (size_t)row0 * ksb;
+  // the wave's column blocks (columns past N: clamped, never stored)
+  const uint8_t* b_base;
+  uint32_t ob[kCB];
+  if constexpr (kLay == SmallWeights::kPacked) b_base = b + (size_t)e * ((size_t)N * Kd);
+  else b_base = b + ((size_t)e * N + (kSwiGLU ? 0 : n0)) * Kd;
+#pragma unroll
+  for (int j = 0; j < kCB; ++j) {
+    const int wr0 = kSwiGLU ? (wid < 2 ? 0 : I) + nt * kGroup + (wid & 1) * 64 + j * 16
+                            : min(n0 + wid * 16 * kCB + j * 16, N - 16);
+    if constexpr (kLay == SmallWeights::kPacked)
+      ob[j] = (uint32_t)(wr0 / 16) * (uint32_t)ksb * 2048u + (uint32_t)lane * 16u;
+    else
+      ob[j] = (uint32_t)((wr0 - (kSwiGLU ? 0 : n0) + (lane & 15)) * Kd + (lane >> 4) * 32);
+  }
+  const int blk = kSwiGLU ? (wid < 2 ? nt : I / kGroup + nt)
+                          : min((n0 + wid * 16 * kCB) / kGroup, NB - 1);
+  const float* sb_row = bs + ((size_t)e * NB + blk) * ksb;
+
+  if (rows <= 16) run_tile<kLay, kE8, kCB, 1, 4>(a_base, s_base, b_base, sb_row, ob, rows, Kd, ksb, smem, tid);
+  else if (rows <= 32) run_tile<kLay, kE8, kCB, 2, 4>(a_base, s_base, b_base, sb_row, ob, rows, Kd, ksb, smem, tid);
+  else if (rows <= 64) run_tile<kLay, kE8, kCB, 4, 2>(a_base, s_base, b_base, sb_row, ob, rows, Kd, ksb, smem, tid);
+  else run_tile<kLay, kE8, kCB, 6, 2>(a_base, s_base, b_base, sb_row, ob, rows, Kd, ksb, smem, tid);
+  __syncthreads();
+
+  if constexpr (kSwiGLU) {
+    // 8 lanes per row, 16 columns each: h = silu(g) * u from the staged bf16
+    // values, amax over the 8 lanes, 16 fp8 bytes per lane
+    for (int idx = tid; idx < rows * 8; idx += kThreads) {
+      const int r = idx >> 3, sub = idx & 7;
+      const uint8_t* rowp = smem + r * kCPitch;
+      float fgt[16], fu[16], h[16];
+      unpack_bf16x8(*(const uint4*)(rowp + sub * 32), fgt);
+      unpack_bf16x8(*(const uint4*)(rowp + sub * 32 + 16), fgt + 8);
+      unpack_bf16x8(*(const uint4*)(rowp + 256 + sub * 32), fu);
+      unpack_bf16x8(*(const uint4*)(rowp + 256 + sub * 32 + 16), fu + 8);
+#pragma unroll
+      for (int i = 0; i < 16; ++i) h[i] = silu32(fgt[i]) * fu[i];
+      const Q16 q = quant16<kE8>(h);
+      const size_t gr = (size_t)(row0 + r);
+      *(uint4*)(hq + gr * I + nt * kGroup + sub * 16) = q.q;
+      if (sub == 0) hs[gr * (I / kGroup) + nt] = q.scale;
+      if (c) {
+        uint16_t* crow = c + gr * N + nt * kGroup + sub * 16;
+        *(uint4*)crow = *(const uint4*)(rowp + sub * 32);
+        *(uint4*)(crow + 8) = *(const uint4*)(rowp + sub * 32 + 16);
+        *(uint4*)(crow + I) = *(const uint4*)(rowp + 256 + sub * 32);
+        *(uint4*)(crow + I + 8) = *(const uint4*)(rowp + 256 + sub * 32 + 16);
+      }
+    }
+  } else {
+    constexpr int kChunks = kBN / 8;  // 16-byte pieces of an output row
+    const int ncols = min(kBN, N - n0);
+    for (int idx = tid; idx < rows * kChunks; idx += kThreads) {
+      const int r = idx / kChunks, ch = idx % kChunks;
+      if (ch * 8 < ncols)
+        *(uint4*)(c + (size_t)(row0 + r) * N + n0 + ch * 8) = *(const uint4*)(smem + r * kCPitch + ch * 16);
+    }
+  }
+}
+
+}  // namespace small
+
+// The line between this kernel and the 256-row ones, on the average rows per
+// expert (the host knows no more).  Up to it an expert's rows mostly fit one
+// 96-row tile and its weights are streamed once; past it the second tile's
+// weights cost more than the 256-row tile's idle MFMAs.  Packed weights, fc1
+// with SwiGLU, 256-row kernel -> this one in us: 75 rows (H 4096, I 14336) 265
+// -> 182, 62 rows (H 2048, I 768) 125 -> 97, 65 rows (H 7168, I 2048) 241 ->
+// 182, but 100 rows of the last 253 -> 246 and their E8M0 form 223 -> 245.
+// Plain weights, whose fragment loads touch 16 lines each: 62 rows (H = I =
+// 2880) 165 -> 146, 97 rows 172 -> 188.  Under Zipf(1.2) loads the averages
+// below the line gain as much (65 rows: 246 -> 204 packed, 261 -> 245 plain),
+// and 88 rows lose (packed E8M0 227 -> 242, plain 269 -> 302).
+bool small_gemm_rows(SmallWeights lay, int E, int R) {
+  return R <= (lay == SmallWeights::kPacked ? 80LL : 64LL) * E;
+}
+
+int small_gemm_launch(SmallWeights lay, bool e8m0, const uint8_t* a, const float* as,
+                      const uint8_t* b, const float* bs, const int32_t* offsets, int E, int R,
+                      int N, int Kdim, uint16_t* c, uint8_t* hq, float* hs, hipStream_t stream) {
+  // at most min(E, R) experts have rows, and each adds at most one partial tile
+  const int live = E < R ? E : R;
+  const long long mt = live + (R - live) / small::kBM;
+  const bool swiglu = hq != nullptr;
+  int cb = 4;
+  if (!swiglu) {
+    // columns per workgroup: narrower while the launch has fewer than two
+    // workgroups per CU
+    while (cb > 1 && live * (long long)((N + 64 * cb - 1) / (64 * cb)) < 512) cb >>= 1;
+  }
+  const long long NT = swiglu ? N / 2 / kGroup : (N + 64 * cb - 1) / (64 * cb);
+  const long long nblk = (mt * NT + 7) / 8 * 8;
+  if (nblk > 0x7fffffffLL) return SMOE_EINVAL_DIM;
+#define SMOE_SG(LAY, E8, SW, CB)                                                                \
+  small::gemm_small_kernel<SmallWeights::LAY, E8, SW, CB>                                        \
+      <<<dim3((unsigned)nblk), dim3(small::kThreads), 0, stream>>>(a, as, b, bs, offsets, E, R, \
+                                                                   N, Kdim, (int)mt, c, hq, hs)
+#define SMOE_SG_CB(LAY, E8)                    \
+  do {                                         \
+    if (swiglu) SMOE_SG(LAY, E8, true, 4);     \
+    else if (cb == 4) SMOE_SG(LAY, E8, false, 4); \
+    else if (cb == 2) SMOE_SG(LAY, E8, false, 2); \
+    else SMOE_SG(LAY, E8, false, 1);           \
+  } while (0)
+  if (lay == SmallWeights::kPlain) SMOE_SG_CB(kPlain, false);
+  else if (e8m0) SMOE_SG_CB(kPacked, true);
+  else SMOE_SG_CB(kPacked, false);
+#undef SMOE_SG_CB
+#undef SMOE_SG
+  SMOE_RETURN_LAUNCH();
+}
+
+}  // namespace smoe

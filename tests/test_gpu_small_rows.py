@@ -1,0 +1,147 @@
+"""The grouped GEMM for few rows per expert (smoe_gemm_small.hip) against the
+256-row kernels, byte for byte: the same operands with unused rows past
+offsets[E], which push the average over the line, take the general path.
+The row counts sit on the edges of the 16-row blocks and of the 96-row tile,
+K on both sides of the load-ahead and of the 64-step scale window, N on
+partial column tiles; more than 256 experts take the tile search's long
+form.  A CPU model checks the tile mapping for valid and malformed offsets."""
+import numpy as np
+import pytest
+import torch
+
+from oracle import smoe_oracle as O
+from smoe import ops
+from smoe import workloads as W
+
+BM = 96
+
+
+# ------------------------------------------------------------- CPU model
+def tiles(R, NT, offsets):
+    """(expert, first row, rows, column tile) of every workgroup that works."""
+    E = len(offsets) - 1
+    live = min(E, R)
+    bound = live + (R - live) // BM
+    cnt = [min(-(-max(0, int(offsets[e + 1]) - int(offsets[e])) // BM), bound) for e in range(E)]
+    total = 0
+    for b in range(0, E, 64):
+        total = min(total + sum(cnt[b:b + 64]), bound)
+    out, n = [], total * NT
+    chunk = (n + 7) // 8
+    for bid in range((bound * NT + 7) // 8 * 8):
+        tl = (bid & 7) * chunk + (bid >> 3)
+        if (bid >> 3) >= chunk or tl >= n:
+            continue
+        mt, first, e = tl // NT, 0, 0
+        while e < E and first + cnt[e] <= mt:
+            first += cnt[e]
+            e += 1
+        q = tl - first * NT
+        nt = q // cnt[e]
+        o0, o1 = int(offsets[e]), int(offsets[e + 1])
+        h = min((-(-(o1 - o0) // cnt[e]) + 15) & ~15, BM)
+        row0 = o0 + (q - nt * cnt[e]) * h
+        rows = min(h, min(o1, R) - row0)
+        if row0 >= 0 and rows > 0:
+            out.append((e, row0, rows, nt))
+    return out
+
+
+def test_tiles_cover_every_row_once():
+    rng = np.random.default_rng(3)
+    for _ in range(200):
+        E = int(rng.integers(1, 300))
+        counts = rng.integers(0, rng.choice([2, 40, 400]), E)
+        counts[rng.random(E) < 0.3] = 0
+        lead = int(rng.integers(0, 5))
+        R = max(1, lead + int(counts.sum()) + int(rng.integers(0, 50)))
+        off = lead + np.concatenate([[0], np.cumsum(counts)])
+        NT = int(rng.integers(1, 4))
+        seen = np.zeros((R, NT), int)
+        for e, row0, rows, nt in tiles(R, NT, off):
+            assert off[e] <= row0 and row0 + rows <= off[e + 1] and rows <= BM
+            seen[row0:row0 + rows, nt] += 1
+        assert (seen[off[0]:off[-1]] == 1).all() and seen.sum() == int(counts.sum()) * NT
+
+
+def test_tiles_stay_in_range_for_malformed_offsets():
+    rng = np.random.default_rng(4)
+    for _ in range(200):
+        E, R = int(rng.integers(1, 9)), int(rng.integers(1, 400))
+        off = int(rng.integers(-300, 300)) + np.concatenate([[0], np.cumsum(rng.integers(-300, 900, E))])
+        for _, row0, rows, _ in tiles(R, 2, off):
+            assert 0 <= row0 and row0 + rows <= R and rows <= BM
+
+
+# ------------------------------------------------------------------- GPU
+def bits(t):
+    return t.contiguous().view(torch.uint8 if t.element_size() == 1 else torch.int16
+                               if t.element_size() == 2 else torch.int32)
+
+
+CASES = [
+    # counts, N, K: tile and block edges; K of 1, 3 and 5 steps, past 64 and 128 steps
+    ([1, 15, 16, 17, 0, 31, 32, 33, 48, 49, 63, 64, 65], 512, 512),
+    ([95, 96, 97, 0, 2, 191, 0, 0, 192, 193, 1, 0, 0, 0, 0, 0], 256, 1024),
+    ([5, 0, 20, 70], 272, 128),
+    ([40, 3], 1040, 640),
+    ([2, 0, 90, 33], 256, 66 * 128),
+    ([33, 7, 0, 60], 256, 132 * 128),
+    ([1], 128, 384),
+    ([3, 0, 1, 100, 0, 17] * 60, 256, 512),
+]
+
+
+def run(xq, xs, w, ws, off, R, e8m0, swiglu, N):
+    """The valid rows' outputs with buffers of R rows; none past offsets[E]
+    is written."""
+    n = int(off[-1])
+    rows = xq.new_empty((R,) + xq.shape[1:])
+    sc = xs.new_empty((R,) + xs.shape[1:])
+    rows.view(torch.uint8).zero_()
+    sc.fill_(1.0)
+    rows.view(torch.uint8)[:n], sc[:n] = xq.view(torch.uint8)[:n], xs[:n]
+    if swiglu:
+        out = ops.grouped_gemm_fp8_swiglu(rows, sc, w, ws, off, save_c1=True, scale="pow2" if e8m0 else "amax")
+        return [bits(o[:n]) for o in out]
+    out = torch.full((R, N), 7.0, dtype=torch.bfloat16, device=xq.device)
+    ops.grouped_gemm_fp8(rows, sc, w, ws, off, out=out, e8m0=e8m0)
+    assert (out[n:].float() == 7.0).all()
+    return [bits(out[:n])]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("counts,N,K", CASES)
+@pytest.mark.parametrize("form", ["plain", "packed", "e8m0"])
+def test_small_rows_equal_the_256_row_kernels(dev, counts, N, K, form):
+    print("[small]", form, len(counts), N, K, flush=True)
+    E, n = len(counts), int(sum(counts))
+    e8m0 = form == "e8m0"
+    if form != "plain" and not (ops.packed_e8m0_ok if e8m0 else ops.packed_gemm_ok)(N, K):
+        with pytest.raises(ValueError):  # refused as before
+            wq = torch.zeros((E, N, K), dtype=torch.uint8, device=dev)
+            ops.grouped_gemm_fp8(torch.zeros((n, K), dtype=torch.uint8, device=dev),
+                                 torch.ones((n, K // 128), device=dev), ops.PackedWeight(wq),
+                                 torch.ones((E, -(-N // 128), K // 128), device=dev),
+                                 W.offsets_from_counts(counts, dev), e8m0=e8m0)
+        return
+    scale = "pow2" if e8m0 else "amax"
+    off = W.offsets_from_counts(counts, dev)
+    x = W.tokens(n, K, device=dev, seed=K + N)
+    xq, xs = ops.quant_rows(x, scale=scale)
+    wq, ws = ops.quantize_weight_blockwise(W.weights(E, N, K, device=dev, seed=N), scale=scale)
+    w = wq if form == "plain" else ops.pack_weight_fp8(wq)
+    big = 81 * E + n  # over the line: the 256-row kernels
+    for swiglu in (False, True):
+        if swiglu and N % 256:
+            continue
+        few = run(xq, xs, w, ws, off, n, e8m0, swiglu, N)
+        for a, b in zip(few, run(xq, xs, w, ws, off, big, e8m0, swiglu, N)):
+            assert torch.equal(a, b), f"swiglu={swiglu}"
+        if not swiglu and K <= 1024 and E < 20:
+            ref = O.grouped_gemm_fp8(xq.view(torch.uint8).cpu().numpy(), xs.cpu().numpy(),
+                                     wq.view(torch.uint8).cpu().numpy(), ws.cpu().numpy(), off.cpu().numpy())
+            got = few[0].view(torch.bfloat16).float().cpu().numpy()
+            # bf16 rounds to 2^-9 of a value, about 1.4e-3 on average
+            d = np.abs(got - ref)
+            assert d.max() <= 1e-2 * np.abs(ref).max() and d.mean() <= 2e-3 * np.abs(ref).mean()
