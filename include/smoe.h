@@ -281,6 +281,15 @@ int smoe_grouped_gemm_fp8_swiglu(const uint8_t* a, const float* as, const uint8_
 int smoe_pack_weight_fp8(const uint8_t* wq, int E, int N, int Kdim, uint8_t* wp, void* stream);
 
 /*
+ * smoe_quantize_weight_blockwise_ex and smoe_pack_weight_fp8 of its result in
+ * one launch: the same wq, ws, and wp [E,N,Kp] bytes (Kp = Kdim padded to a
+ * multiple of 128).  Replaces the same weight-cache refresh
+ * (summary/fp8_expert_gemm_optimization.md:133-143).
+ */
+int smoe_quantize_pack_weight(const uint16_t* w, int E, int N, int Kdim, uint8_t* wq, float* ws,
+                              uint8_t* wp, int scale_mode, void* stream);
+
+/*
  * smoe_grouped_gemm_fp8 on packed weights (smoe_pack_weight_fp8): the same
  * c [R,N] bf16 (bit for bit whenever each 128-wide K block's products sum
  * exactly in fp32; else within the last bf16 bit), from a kernel that loads each wave's weights
@@ -432,6 +441,14 @@ int smoe_quant_rows_1x128_ex(const uint16_t* x, int M, int C, uint8_t* q, float*
  */
 int smoe_transpose_blockwise_fp8(const uint8_t* wq, const float* ws, int E, int N, int Kdim,
                                  uint8_t* wqT, float* wsT, void* stream);
+
+/*
+ * smoe_transpose_blockwise_fp8 and smoe_pack_weight_fp8 of its result in one
+ * launch: wpT [E,Kdim,Np] bytes in fragment order, and wsT.  Replaces the same
+ * weight cache (summary/fp8_expert_gemm_optimization.md:133-143).
+ */
+int smoe_transpose_pack_fp8(const uint8_t* wq, const float* ws, int E, int N, int Kdim,
+                            uint8_t* wpT, float* wsT, void* stream);
 
 /*
  * Transposed 128x1 column quantisation of x [R,C] bf16 whose rows are the

@@ -214,16 +214,23 @@ __global__ __launch_bounds__(256) void swiglu_quant_kernel(const uint16_t* __res
 }
 
 // ------------------------------------------------- weight 128x128 blocks
-// One 256-thread workgroup per 128x128 block.  Thread t owns 8 chunks of 8
-// bf16 (chunk j*256+t -> block row chunk/16, column (chunk%16)*8).  w is
+// One 256-thread workgroup per 128x128 block.  Thread t owns 4 chunks of 16
+// bf16 (chunk j*256+t -> block row chunk/8, column (chunk%8)*16).  w is
 // [E, N, Kd] bf16; wq is [E, N, Kp] with Kp = pad128(Kd), ws [E, NB, Kp/128]
 // with NB = ceil(N/128).  Rows past N and columns past Kd of an edge block
-// are zeros (not read); padding columns are written as byte 0.
-template <bool kPow2 = false>
+// are zeros (not read); padding columns are written as byte 0.  kPack: the
+// same bytes also go to wp in MFMA fragment order (smoe_pack_weight_fp8);
+// a wave's store fills whole 128-byte lines of it (8 rows x 16 bytes), so the
+// packed copy costs its write alone.  Bound by HBM; the stores are
+// non-temporal (cached ones 7% slower).  E 128, N 1536, K 2048: 398 us for the
+// quantiser and a repacking launch, 288 in one (5.6 TB/s); E 32, N 5760, K
+// 2880 E8M0: 501 -> 373.
+template <bool kPow2, bool kPack>
 __global__ __launch_bounds__(256) void quant_weight_kernel(const uint16_t* __restrict__ w,
                                                            int N, int Kd,
                                                            uint8_t* __restrict__ wq,
-                                                           float* __restrict__ ws) {
+                                                           float* __restrict__ ws,
+                                                           uint8_t* __restrict__ wp) {
   __shared__ float wmax[4];
   const int Kp = pad128(Kd);
   const int nb = (N + kGroup - 1) / kGroup, kb = Kp / kGroup;
@@ -232,20 +239,21 @@ __global__ __launch_bounds__(256) void quant_weight_kernel(const uint16_t* __res
   const int rem = blk - e * nb * kb;
   const int bn = rem / kb, bk = rem - bn * kb;
   const int r0 = bn * kGroup, k0 = bk * kGroup;
-  float f[8][8];
+  float f[4][16];
   float amax = 0.0f;
 #pragma unroll
-  for (int j = 0; j < 8; ++j) {
+  for (int j = 0; j < 4; ++j) {
     const int ch = j * 256 + threadIdx.x;
-    const int row = ch >> 4, col = (ch & 15) * 8;
+    const int row = ch >> 3, col = (ch & 7) * 16;
     const bool ok = r0 + row < N && k0 + col < Kd;
-    // unconditional load (an edge chunk re-reads the block's first element)
-    const uint16_t* src = w + ((size_t)e * N + r0 + (ok ? row : 0)) * Kd + k0 + (ok ? col : 0);
-    uint4 v = *(const uint4*)src;
-    if (!ok) v = make_uint4(0, 0, 0, 0);
-    unpack_bf16x8(v, f[j]);
+    // unconditional load (an edge chunk re-reads the block's first elements)
+    const uint4* src = (const uint4*)(w + ((size_t)e * N + r0 + (ok ? row : 0)) * Kd + k0 + (ok ? col : 0));
+    uint4 a = src[0], b = src[1];
+    if (!ok) a = b = make_uint4(0, 0, 0, 0);
+    unpack_bf16x8(a, f[j]);
+    unpack_bf16x8(b, f[j] + 8);
 #pragma unroll
-    for (int i = 0; i < 8; ++i) amax = fmaxf(amax, fabsf(f[j][i]));
+    for (int i = 0; i < 16; ++i) amax = fmaxf(amax, fabsf(f[j][i]));
   }
   amax = wave_max(amax);
   if ((threadIdx.x & 63) == 0) wmax[threadIdx.x >> 6] = amax;
@@ -254,15 +262,21 @@ __global__ __launch_bounds__(256) void quant_weight_kernel(const uint16_t* __res
   const float s = scale_of<kPow2>(amax);
   const QDiv d = qdiv_setup_t<kPow2>(s);
 #pragma unroll
-  for (int j = 0; j < 8; ++j) {
+  for (int j = 0; j < 4; ++j) {
     const int ch = j * 256 + threadIdx.x;
-    const int row = ch >> 4, col = (ch & 15) * 8;
-    const uint32_t lo = e4m3_pack4(quot_t<kPow2>(f[j][0], d), quot_t<kPow2>(f[j][1], d),
-                                   quot_t<kPow2>(f[j][2], d), quot_t<kPow2>(f[j][3], d));
-    const uint32_t hi = e4m3_pack4(quot_t<kPow2>(f[j][4], d), quot_t<kPow2>(f[j][5], d),
-                                   quot_t<kPow2>(f[j][6], d), quot_t<kPow2>(f[j][7], d));
-    if (r0 + row < N)
-      *(uint2*)(wq + ((size_t)e * N + r0 + row) * Kp + k0 + col) = make_uint2(lo, hi);
+    const int row = ch >> 3, q = ch & 7;
+    uint32_t o[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+      o[i] = e4m3_pack4(quot_t<kPow2>(f[j][4 * i], d), quot_t<kPow2>(f[j][4 * i + 1], d),
+                        quot_t<kPow2>(f[j][4 * i + 2], d), quot_t<kPow2>(f[j][4 * i + 3], d));
+    if (r0 + row < N) {
+      const uint4 v = make_uint4(o[0], o[1], o[2], o[3]);
+      store16<true>(wq + ((size_t)e * N + r0 + row) * Kp + k0 + q * 16, v);
+      if constexpr (kPack)  // half q/4, lane (q%4)*16 + row%16 of 16-row block (r0 + row)/16
+        store16<true>(wp + (((size_t)e * (N / 16) + (r0 + row) / 16) * kb + bk) * 2048 + (q >> 2) * 1024 +
+                  ((q & 3) * 16 + (row & 15)) * 16, v);
+    }
   }
   if (threadIdx.x == 0) ws[((size_t)e * nb + bn) * kb + bk] = s;
 }
@@ -540,9 +554,9 @@ extern "C" int smoe_swiglu_quant(const uint16_t* c1, int R, int I, uint8_t* hq, 
   return smoe_swiglu_quant_ex(c1, R, I, hq, hs, nullptr, SMOE_SCALE_AMAX, stream);
 }
 
-extern "C" int smoe_quantize_weight_blockwise_ex(const uint16_t* w, int E, int N, int Kdim,
-                                                 uint8_t* wq, float* ws, int scale_mode,
-                                                 void* stream) {
+namespace {
+int quant_weight_launch(const uint16_t* w, int E, int N, int Kdim, uint8_t* wq, float* ws,
+                        uint8_t* wp, int scale_mode, hipStream_t s) {
   if (N <= 0 || Kdim <= 0) return SMOE_EINVAL_DIM;
   if (E <= 0 || E > SMOE_MAX_EXPERTS) return SMOE_EINVAL_EXPERTS;
   if (N % kLane || Kdim % kLane) return SMOE_EINVAL_ALIGN128;
@@ -553,12 +567,24 @@ extern "C" int smoe_quantize_weight_blockwise_ex(const uint16_t* w, int E, int N
   const long long blocks = (long long)E * ((N + kGroup - 1) / kGroup) * (pad128(Kdim) / kGroup);
   if (blocks > 0x7fffffffLL) return SMOE_EINVAL_DIM;
   const dim3 grid((unsigned)blocks), block(256);
-  hipStream_t s = (hipStream_t)stream;
-  if (scale_mode == SMOE_SCALE_POW2)
-    quant_weight_kernel<true><<<grid, block, 0, s>>>(w, N, Kdim, wq, ws);
-  else
-    quant_weight_kernel<false><<<grid, block, 0, s>>>(w, N, Kdim, wq, ws);
+#define SMOE_QW(P2, PK) quant_weight_kernel<P2, PK><<<grid, block, 0, s>>>(w, N, Kdim, wq, ws, wp)
+  if (scale_mode == SMOE_SCALE_POW2) { if (wp) SMOE_QW(true, true); else SMOE_QW(true, false); }
+  else { if (wp) SMOE_QW(false, true); else SMOE_QW(false, false); }
+#undef SMOE_QW
   SMOE_RETURN_LAUNCH();
+}
+}  // namespace
+
+extern "C" int smoe_quantize_weight_blockwise_ex(const uint16_t* w, int E, int N, int Kdim,
+                                                 uint8_t* wq, float* ws, int scale_mode,
+                                                 void* stream) {
+  return quant_weight_launch(w, E, N, Kdim, wq, ws, nullptr, scale_mode, (hipStream_t)stream);
+}
+
+extern "C" int smoe_quantize_pack_weight(const uint16_t* w, int E, int N, int Kdim, uint8_t* wq,
+                                         float* ws, uint8_t* wp, int scale_mode, void* stream) {
+  SMOE_CHECK_PTR(wp);
+  return quant_weight_launch(w, E, N, Kdim, wq, ws, wp, scale_mode, (hipStream_t)stream);
 }
 
 extern "C" int smoe_quantize_weight_blockwise(const uint16_t* w, int E, int N, int Kdim,

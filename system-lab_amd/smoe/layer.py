@@ -167,22 +167,27 @@ class SimpleMoE(nn.Module):
     @torch.no_grad()
     def refresh_fp8_cache(self):
         rs = self._row_scale
-        w1q, w1s = ops.quantize_weight_blockwise(self.w1.detach().to(torch.bfloat16).contiguous(), rs)
-        w2q, w2s = ops.quantize_weight_blockwise(self.w2.detach().to(torch.bfloat16).contiguous(), rs)
-        self._fp8 = (w1q, w1s, w2q, w2s)
+        fp8, gemm = [], []
+        for p in (self.w1, self.w2):
+            w = p.detach().to(torch.bfloat16).contiguous()
+            if self._packs(w.shape[1], ops.pad128(w.shape[2])):
+                wq, ws, wg = ops.quantize_pack_weight(w, rs)
+            else:
+                wq, ws = ops.quantize_weight_blockwise(w, rs)
+                wg = wq
+            fp8 += [wq, ws]
+            gemm += [wg, ws]
+        self._fp8, self._gemm = tuple(fp8), tuple(gemm)
         self._fp8_key = self._weights_key()
-        self._gemm = (self._for_gemm(w1q), w1s, self._for_gemm(w2q), w2s)
         self._gemm_t = None
         return self._fp8
 
-    def _for_gemm(self, wq):
-        """The form the GEMM ops take: packed in MFMA fragment order where the
-        register-loaded kernel covers the shape (K a multiple of 512, or for
-        the E8M0 recipe of 128 from 512 up; the same bytes out, faster), else
-        the plain [E, N, K] weights."""
-        E, N, Kd = wq.shape
-        ok = ops.packed_e8m0_ok if self._pow2 else ops.packed_gemm_ok
-        return ops.pack_weight_fp8(wq) if ok(N, Kd) else wq
+    def _packs(self, N: int, Kd: int) -> bool:
+        """Whether the GEMM ops take an [E, N, Kd] fp8 weight packed in MFMA
+        fragment order: where the register-loaded kernel covers the shape (K a
+        multiple of 512, or for the E8M0 recipe of 128 from 512 up; the same
+        bytes out, faster).  Others stay plain."""
+        return (ops.packed_e8m0_ok if self._pow2 else ops.packed_gemm_ok)(N, Kd)
 
     def fp8_weights(self):
         """(w1q, w1s, w2q, w2s), re-quantised when w1 or w2 changed since the
@@ -197,10 +202,13 @@ class SimpleMoE(nn.Module):
         ``gemm_weights_t``)."""
         return self._transposed(self.fp8_weights())
 
-    def _transposed(self, fp8):
-        w1q, w1s, w2q, w2s = fp8
-        return (ops.transpose_blockwise(w1q, w1s, k=self.hidden)
-                + ops.transpose_blockwise(w2q, w2s, k=self.intermediate))
+    def _transposed(self, fp8, gemm: bool = False):
+        """Transposes of fp8 weights: plain, or (gemm) as the GEMM ops take them."""
+        out = ()
+        for wq, ws, k in ((fp8[0], fp8[1], self.hidden), (fp8[2], fp8[3], self.intermediate)):
+            pack = gemm and self._packs(k, ops.pad128(wq.shape[1]))
+            out += ops.transpose_blockwise(wq, ws, k=k, pack=pack)
+        return out
 
     def gemm_weights(self):
         """(w1, w1s, w2, w2s) as the forward GEMMs take them: fp8_weights()
@@ -215,11 +223,9 @@ class SimpleMoE(nn.Module):
         whose transposes are computed and not cached."""
         cur = self.fp8_weights()
         if fp8 is not None and fp8 is not cur:
-            w1tq, w1ts, w2tq, w2ts = self._transposed(fp8)
-            return (self._for_gemm(w1tq), w1ts, self._for_gemm(w2tq), w2ts)
+            return self._transposed(fp8, gemm=True)
         if self._gemm_t is None:
-            w1tq, w1ts, w2tq, w2ts = self._transposed(cur)
-            self._gemm_t = (self._for_gemm(w1tq), w1ts, self._for_gemm(w2tq), w2ts)
+            self._gemm_t = self._transposed(cur, gemm=True)
         return self._gemm_t
 
     def forward(self, x: torch.Tensor, logits: torch.Tensor | None = None,

@@ -351,6 +351,27 @@ def pack_weight_fp8(wq: torch.Tensor) -> PackedWeight:
     return PackedWeight(wp)
 
 
+def _packable(N: int, Kd: int) -> bool:
+    return packed_gemm_ok(N, Kd) or packed_e8m0_ok(N, Kd)
+
+
+def quantize_pack_weight(w: torch.Tensor, scale: str = "amax"):
+    """``quantize_weight_blockwise`` and ``pack_weight_fp8`` of its result from
+    one read of w: -> (wq, ws, PackedWeight), the same bytes.  Raises like
+    ``pack_weight_fp8`` when no packed kernel covers the shape."""
+    mode = _scale(scale)
+    _check(w, "w", (torch.bfloat16,), 3)
+    E, N, Kd = w.shape
+    Kp = pad128(Kd)
+    if not _packable(N, Kp):
+        raise ValueError(f"no packed kernel covers N={N}, K={Kp}")
+    wq = torch.empty((E, N, Kp), dtype=FP8, device=w.device)
+    ws = torch.empty((E, nblocks(N), nblocks(Kd)), dtype=torch.float32, device=w.device)
+    wp = torch.empty((E, N, Kp), dtype=torch.uint8, device=w.device)
+    _C.call("smoe_quantize_pack_weight", _ptr(w), E, N, Kd, _ptr(wq), _ptr(ws), _ptr(wp), mode, _stream())
+    return wq, ws, PackedWeight(wp)
+
+
 def _weight(wq, name):
     """(tensor, packed?) of a GEMM weight argument."""
     if isinstance(wq, PackedWeight):
@@ -521,11 +542,13 @@ def quant_rows(x: torch.Tensor, scale: str = "amax"):
     return q, s
 
 
-def transpose_blockwise(wq: torch.Tensor, ws: torch.Tensor, k: int | None = None):
+def transpose_blockwise(wq: torch.Tensor, ws: torch.Tensor, k: int | None = None,
+                        pack: bool = False):
     """[E,N,Kp] fp8 + [E,NB,KB] -> [E,K,pad128(N)] + [E,KB,NB] (dgrad
     weights; blockwise quantisation commutes with the transpose).  ``k`` is
     the true K when wq's pitch Kp = pad128(K) holds padding (default Kp);
-    the result's padding columns past N are 0."""
+    the result's padding columns past N are 0.  ``pack``: the transposed
+    weight comes as the PackedWeight of it (``pack_weight_fp8``) instead."""
     _check(wq, "wq", (FP8, torch.uint8), 3)
     _check(ws, "ws", (torch.float32,), 3)
     E, N, Kp = wq.shape
@@ -534,8 +557,14 @@ def transpose_blockwise(wq: torch.Tensor, ws: torch.Tensor, k: int | None = None
         raise ValueError(f"wq [{E}, {N}, {Kp}] is not the padded form of a K = {Kd} weight")
     if tuple(ws.shape) != (E, nblocks(N), Kp // GROUP):
         raise ValueError(f"ws must be [{E}, {nblocks(N)}, {Kp // GROUP}] for wq {tuple(wq.shape)}")
-    wqT = torch.empty((E, Kd, pad128(N)), dtype=FP8, device=wq.device)
+    if pack and not _packable(Kd, pad128(N)):
+        raise ValueError(f"no packed kernel covers N={Kd}, K={pad128(N)}")
+    wqT = torch.empty((E, Kd, pad128(N)), dtype=torch.uint8 if pack else FP8, device=wq.device)
     wsT = torch.empty((E, Kp // GROUP, nblocks(N)), dtype=torch.float32, device=wq.device)
+    if pack:
+        _C.call("smoe_transpose_pack_fp8", _ptr(_bytes(wq)), _ptr(ws), E, N, Kd, _ptr(wqT), _ptr(wsT),
+                _stream())
+        return PackedWeight(wqT), wsT
     _C.call("smoe_transpose_blockwise_fp8", _ptr(_bytes(wq)), _ptr(ws), E, N, Kd,
             _ptr(wqT), _ptr(wsT), _stream())
     return wqT, wsT
