@@ -188,6 +188,28 @@ int smoe_dispatch_quant(const uint16_t* x, const int32_t* topk_idx, int T, int H
                         size_t ws_bytes, void* stream);
 
 /*
+ * Router, expert sort and permute + 1x128 quantisation of one batch: the
+ * outputs of smoe_route_topk_sort then smoe_permute_quant_ex, byte for byte;
+ * batches of up to 256 tokens and 2048 pairs in one or two launches.  With
+ * logits NULL the logits are x . w_gate [H,E] f32 (fp32 products of the bf16
+ * tokens, summed in fp32), for the batches smoe_gate_fused_ok accepts.
+ * ws: smoe_route_dispatch_workspace_size bytes, status word first.
+ * smoe_gate_logits writes the same logits [T,E] f32 (ws as above; its status
+ * word is left alone).
+ * Replaces the gate linear, router and Dispatcher.permute of one step
+ * (moe/MoE_detailed_computation_dataflow.md:53-66; moe/MegatronCore_MoE_reading_notes.md:94-99).
+ */
+int smoe_gate_fused_ok(int T, int H, int E, int K);
+size_t smoe_route_dispatch_workspace_size(int T, int H, int E, int K);
+int smoe_gate_logits(const uint16_t* x, const float* w_gate, int T, int H, int E, int K,
+                     float* logits, void* ws, size_t ws_bytes, void* stream);
+int smoe_route_dispatch(const uint16_t* x, const float* logits, const float* w_gate,
+                        const float* bias, int T, int H, int E, int K, int32_t* topk_idx,
+                        float* topk_w, int32_t* row_map, int32_t* inv_map, int32_t* counts,
+                        int32_t* offsets, uint8_t* xq, float* xs, int scale_mode, void* ws,
+                        size_t ws_bytes, void* stream);
+
+/*
  * 128x128 blockwise fp8 weight quantisation.  w [E,N,Kdim] bf16 (Kdim
  * contiguous, "NK" layout) -> wq [E,N,Kp] u8, ws [E,ceil(N/128),Kp/128] f32
  * with Kp = Kdim padded to a multiple of 128 (padding columns 0).

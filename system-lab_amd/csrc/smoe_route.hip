@@ -266,18 +266,51 @@ __device__ __forceinline__ TokenRoute<kLPT, kNV> route_token(const float* __rest
   return r;
 }
 
-// Router only: kLPT lanes per token, 256 threads.
-template <int kLPT, int kNV>
+// out[i] = the sum over s of part[s * stride + i], in order, for i < n: the
+// logits of some tokens from the gating linear's slices, by a workgroup.
+__device__ __forceinline__ void sum_parts(const float* __restrict__ part, int nsplit, size_t stride,
+                                          int n, float* out) {
+  // two values and eight slices of each in flight
+  for (int i = threadIdx.x; i < n; i += 512) {
+    const int k = min(i + 256, n - 1);
+    float a = 0.0f, b = 0.0f;
+    for (int s0 = 0; s0 < nsplit; s0 += 8) {
+      float va[8], vb[8];
+#pragma unroll
+      for (int u = 0; u < 8; ++u) {
+        const float* p = part + (size_t)min(s0 + u, nsplit - 1) * stride;
+        va[u] = p[i];
+        vb[u] = p[k];
+      }
+#pragma unroll
+      for (int u = 0; u < 8; ++u) {
+        a = s0 + u < nsplit ? a + va[u] : a;
+        b = s0 + u < nsplit ? b + vb[u] : b;
+      }
+    }
+    out[i] = a;
+    if (i + 256 < n) out[k] = b;
+  }
+  __syncthreads();
+}
+
+// Router only: kLPT lanes per token, 256 threads.  kParts: logits are nsplit
+// slices [T][E] to be added up (gate_partial_kernel), E <= 256.
+template <int kLPT, int kNV, bool kParts = false>
 __global__ __launch_bounds__(256) void router_topk_kernel(
     const float* __restrict__ logits, const float* __restrict__ bias, int T, int E, int K,
-    int32_t* __restrict__ topk_idx, float* __restrict__ topk_w) {
+    int32_t* __restrict__ topk_idx, float* __restrict__ topk_w, int nsplit) {
   __shared__ float ptab[256 * kNV];  // E <= kLPT*kNV probabilities per token group
   const int i = threadIdx.x & (kLPT - 1);
   const int g = threadIdx.x / kLPT;
-  const int t = blockIdx.x * (256 / kLPT) + g;
+  const int t0 = blockIdx.x * (256 / kLPT), t = t0 + g;
+  __shared__ float lg[kParts ? 256 * kNV : 1];
+  if constexpr (kParts)
+    sum_parts(logits + (size_t)t0 * E, nsplit, (size_t)T * E, min(256 / kLPT, T - t0) * E, lg);
   if (t >= T) return;  // whole token groups leave; no workgroup barrier below
+  const float* row = kParts ? lg + g * E : logits + (size_t)t * E;
   const TokenRoute<kLPT, kNV> r =
-      route_token<kLPT, kNV>(logits + (size_t)t * E, bias, E, K, i, ptab + g * kLPT * kNV);
+      route_token<kLPT, kNV>(row, bias, E, K, i, ptab + g * kLPT * kNV);
 #pragma unroll
   for (int s = 0; s < 2; ++s) {
     const int k = s * kLPT + i;
@@ -646,6 +679,211 @@ __global__ __launch_bounds__(256) void route_rank_wg_kernel(const int32_t* __res
   }
 }
 
+// ------------------------------------------- small batches (decode steps)
+// The gating linear of a few tokens: part[s][t][e] = sum over the s-th H
+// slice of x[t][h] * w[h][e], fp32 products of the bf16 tokens added in fp32.
+// Bound by launch and latency: w_gate is 1 MB at H 2048, E 128.  A workgroup
+// takes 8 tokens x one slice (held in LDS as fp32) x 64 experts.  kEL lanes
+// of a wave hold an expert each, the 64/kEL lane groups and the 4 waves take rows of w in
+// turn (a wave reads 64/kEL whole rows at once, 32 loads in flight), and their
+// sums meet in LDS in a fixed order.
+constexpr int kGateT = 8, kGateMaxE = 256, kGateMaxSlice = 1024;
+// A library product (and the copy of x to fp32 before it) catches up where
+// the fp32 FMAs outweigh its start: with the routing, H 2048, E 128: 24.4 -> 15.5
+// us at 1 token, 27.4 -> 23.1 at 128, 28.3 -> 28.0 at 256; H 7168, E 256: 40.6 ->
+// 29.7 at 1, 42.4 -> 38.8 at 16, 42.9 -> 43.1 at 33; H 4096, E 8, 32 tokens: 26.8 ->
+// 10.1.
+constexpr long long kGateMaxWork = 1LL << 25;  // T * H * E
+template <int kEL>
+__global__ __launch_bounds__(256) void gate_partial_kernel(const uint16_t* __restrict__ x,
+                                                           const float* __restrict__ w, int T,
+                                                           int H, int E, int slice,
+                                                           float* __restrict__ part) {
+  constexpr int kRG = 256 / kEL;  // row groups
+  extern __shared__ float xl[];   // [slice][kGateT], then the groups' sums
+  const int tid = threadIdx.x;
+  const int el = tid % kEL, rg = tid / kEL, e0 = blockIdx.z * 64;
+  const int t0 = blockIdx.x * kGateT, s = blockIdx.y;
+  const int h0 = s * slice, n = min(H - h0, slice);
+  {
+    const int t = tid >> 5;  // 32 threads a token, 8 columns each
+    const uint16_t* xr = x + (size_t)min(t0 + t, T - 1) * H + h0;
+    for (int c = (tid & 31) * 8; c < n; c += 256) {
+      float f[8];
+      unpack_bf16x8(*(const uint4*)(xr + c), f);
+#pragma unroll
+      for (int i = 0; i < 8; ++i) xl[(c + i) * kGateT + t] = f[i];
+    }
+  }
+  __syncthreads();
+  float acc[kGateT];
+#pragma unroll
+  for (int t = 0; t < kGateT; ++t) acc[t] = 0.0f;
+  auto rows = [&](int b, auto u_) __attribute__((always_inline)) {
+    constexpr int kU = decltype(u_)::value;  // rows in flight
+    float wt[kU];
+#pragma unroll
+    for (int u = 0; u < kU; ++u) wt[u] = w[(size_t)(h0 + b + u * kRG) * E + min(e0 + el, E - 1)];
+#pragma unroll
+    for (int u = 0; u < kU; ++u) {
+      const float* xr = xl + (b + u * kRG) * kGateT;
+#pragma unroll
+      for (int t = 0; t < kGateT; ++t) acc[t] = __builtin_fmaf(xr[t], wt[u], acc[t]);
+    }
+  };
+  int b = rg;
+  for (; b + 31 * kRG < n; b += 32 * kRG) rows(b, std::integral_constant<int, 32>{});
+  for (; b + 3 * kRG < n; b += 4 * kRG) rows(b, std::integral_constant<int, 4>{});
+  for (; b < n; b += kRG) rows(b, std::integral_constant<int, 1>{});
+  __syncthreads();
+  float* red = xl;  // [row group][token][expert]
+#pragma unroll
+  for (int t = 0; t < kGateT; ++t) red[(rg * kGateT + t) * kEL + el] = acc[t];
+  __syncthreads();
+  for (int i = tid; i < kGateT * kEL; i += 256) {
+    const int t = i / kEL, e = e0 + i % kEL;
+    if (t0 + t >= T || e >= E) continue;
+    float a = red[i];
+#pragma unroll
+    for (int g = 1; g < kRG; ++g) a = a + red[g * kGateT * kEL + i];
+    part[((size_t)s * T + t0 + t) * E + e] = a;
+  }
+}
+
+// The logits themselves, added up as the routers add them.
+__global__ __launch_bounds__(256) void gate_sum_kernel(const float* __restrict__ part, int nsplit,
+                                                       int n, float* __restrict__ logits) {
+  const int i0 = blockIdx.x * 512;
+  sum_parts(part + i0, nsplit, (size_t)n, min(512, n - i0), logits + i0);
+}
+
+// Sort, permute and 1x128 quantisation of a small batch in one launch: one
+// workgroup per token.  R = T*K ids are few, so every workgroup counts all
+// of them per expert in LDS (and those before its token apart), which gives
+// it the offsets and its K rows without a histogram in memory or a second
+// pass; it then quantises its token (loaded before all that) into them.
+// kRoute: the batch is routed here too, by every workgroup for itself (16
+// tokens a pass).  The order is that of route_sort, the bytes those of
+// permute_quant.
+template <int kLPT, int kNV, bool kRoute, bool kParts, bool kPow2>
+__global__ __launch_bounds__(256) void dispatch_small_kernel(
+    const float* __restrict__ logits, int nsplit, const float* __restrict__ bias,
+    const uint16_t* __restrict__ x, int T, int E, int K, int H, int32_t* __restrict__ topk_idx,
+    float* __restrict__ topk_w, int32_t* __restrict__ row_map, int32_t* __restrict__ inv_map,
+    int32_t* __restrict__ counts, int32_t* __restrict__ offsets, int32_t* __restrict__ status,
+    uint8_t* __restrict__ xq, float* __restrict__ xs) {
+  extern __shared__ int32_t sh[];  // all[E], before[E]; kRoute: ids[R], logits [T][E] (kParts)
+  __shared__ float ptab[kRoute ? 256 * kNV : 1];
+  __shared__ int32_t wtot[4], row[32];
+  int32_t *all = sh, *before = sh + E, *ids = sh + 2 * E;
+  const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
+  const int t = blockIdx.x, R = T * K, p0 = t * K;
+  const int Hp = pad128(H), G = Hp / kGroup;
+  const int sub = lane & 7, gl = lane >> 3;
+  const uint16_t* xrow = x + (size_t)t * H;
+  // wave w quantises 1024-column chunks w, w + 4, ...; the first two are
+  // loaded now (a lane past H reads column 0 and is zeroed)
+  typedef uint32_t v4u __attribute__((ext_vector_type(4)));
+  auto load = [&](int c, v4u& a, v4u& b) {
+    const int col = (c * 8 + gl) * kGroup + sub * kLane;
+    const v4u* src = (const v4u*)(xrow + (col < H ? col : 0));
+    a = src[0];
+    b = src[1];
+    if (col >= H) a = b = v4u{0u, 0u, 0u, 0u};
+  };
+  v4u a0, b0, a1, b1;
+  load(wv, a0, b0);
+  load(wv + 4, a1, b1);
+  for (int e = tid; e < 2 * E; e += 256) sh[e] = 0;
+  if constexpr (kRoute) {
+    const int i = tid & (kLPT - 1), g = tid / kLPT;
+    float* lg = (float*)(ids + R);
+    if constexpr (kParts) sum_parts(logits, nsplit, (size_t)T * E, T * E, lg);
+    for (int tt = g; tt < T; tt += 256 / kLPT) {
+      const float* lrow = kParts ? lg + tt * E : logits + (size_t)tt * E;
+      const TokenRoute<kLPT, kNV> r =
+          route_token<kLPT, kNV>(lrow, bias, E, K, i, ptab + g * kLPT * kNV);
+#pragma unroll
+      for (int s = 0; s < 2; ++s) {
+        const int k = s * kLPT + i;
+        if (k < K) {
+          ids[tt * K + k] = r.id[s];
+          if (tt == t) {
+            topk_idx[p0 + k] = r.id[s];
+            topk_w[p0 + k] = r.w[s];
+          }
+        }
+      }
+    }
+  } else {
+    ids = topk_idx;
+  }
+  __syncthreads();
+  for (int p = tid; p < R; p += 256) {
+    const int e = ids[p];
+    if ((unsigned)e < (unsigned)E) {
+      atomicAdd(&all[e], 1);
+      if (p < p0) atomicAdd(&before[e], 1);
+    }
+  }
+  __syncthreads();
+  // offsets = exclusive scan of the counts (each thread owns up to 4 experts)
+  const int per = (E + 255) / 256;
+  int run = 0;
+  for (int i = 0; i < per; ++i) run += tid * per + i < E ? all[tid * per + i] : 0;
+  const int inc = wave_incl_scan(run, lane);
+  if (lane == kWave - 1) wtot[wv] = inc;
+  __syncthreads();
+  int ex = inc - run;
+  for (int j = 0; j < wv; ++j) ex += wtot[j];
+  for (int i = 0; i < per; ++i) {
+    const int e = tid * per + i;
+    if (e < E) {
+      before[e] += ex;
+      if (t == 0) {
+        offsets[e] = ex;
+        counts[e] = all[e];
+      }
+      ex += all[e];
+    }
+  }
+  if (t == 0 && tid == 0) {
+    const int total = wtot[0] + wtot[1] + wtot[2] + wtot[3];
+    offsets[E] = total;
+    *status = R - total;  // pairs dropped for an id outside [0, E)
+  }
+  __syncthreads();
+  if (tid < K) {
+    const int e = ids[p0 + tid];
+    int r = -1;
+    if ((unsigned)e < (unsigned)E) {
+      r = before[e];
+      for (int k = 0; k < tid; ++k) r += ids[p0 + k] == e;
+      row_map[r] = p0 + tid;
+    }
+    inv_map[p0 + tid] = r;
+    row[tid] = r;
+  }
+  __syncthreads();
+  for (int c = wv; c * 8 < G; c += 4) {
+    float f[16];
+    unpack_bf16x8(make_uint4(a0.x, a0.y, a0.z, a0.w), f);
+    unpack_bf16x8(make_uint4(b0.x, b0.y, b0.z, b0.w), f + 8);
+    a0 = a1;
+    b0 = b1;
+    load(c + 8, a1, b1);
+    const Q16 q = quant16_bf16<kPow2>(f);
+    const int gr = c * 8 + gl;
+    for (int k = 0; k < K; ++k) {
+      const int r = row[k];
+      if ((unsigned)r < (unsigned)R && gr < G) {
+        *(uint4*)(xq + (size_t)r * Hp + gr * kGroup + sub * kLane) = q.q;
+        if (sub == 0) xs[(size_t)r * G + gr] = q.scale;
+      }
+    }
+  }
+}
+
 static inline int seg_count(int R, int seg = kSeg) { return (R + seg - 1) / seg; }
 
 }  // namespace smoe
@@ -683,7 +921,7 @@ extern "C" int smoe_router_topk(const float* logits, const float* bias, int T, i
   hipStream_t s = (hipStream_t)stream;
 #define SMOE_ROUTER(LPT, NV)                                                          \
   router_topk_kernel<LPT, NV><<<dim3((T + 256 / LPT - 1) / (256 / LPT)), dim3(256), 0, s>>>( \
-      logits, bias, T, E, K, topk_idx, topk_w)
+      logits, bias, T, E, K, topk_idx, topk_w, 1)
   SMOE_ROUTE_DISPATCH(E, SMOE_ROUTER);
 #undef SMOE_ROUTER
   SMOE_RETURN_LAUNCH();
@@ -799,6 +1037,151 @@ extern "C" int smoe_route_topk_sort(const float* logits, const float* bias, int 
   SMOE_ROUTE_DISPATCH(E, SMOE_RHIST);
 #undef SMOE_RHIST
   sort_tail<kSegR>(topk_idx, R, E, nseg, row_map, inv_map, counts, offsets, ws, s);
+  SMOE_RETURN_LAUNCH();
+}
+
+// ------------------------------------------------------- route + dispatch
+namespace {
+// The small-batch kernel serves up to 256 tokens and 2048 pairs: every
+// workgroup walks all pairs, so its work grows with their square.  Router +
+// sort + permute in four launches against it, us in a captured queue of calls:
+// H 2048, E 128, top-8: 13.1 -> 7.7 at 1 token, 15.8 -> 11.1 at 128, 16.0 ->
+// 12.4 at 256; H 7168, E 256, top-8: 16.3 -> 10.5 and 21.5 -> 17.1; H 4096, E 8,
+// top-2: 10.5 -> 4.3 and 14.4 -> 6.8.
+bool dispatch_small(int T, int K) { return T <= 256 && (long long)T * K <= 2048; }
+// Routing inside it costs every workgroup a pass per 16 tokens, longer with
+// more experts: the second pass pays up to 32 experts (32 tokens, E 8: 5.5 us
+// inside, 6.0 with a router launch; E 32: 6.7 and 6.8; E 64: 8.7 and 7.9).
+bool route_inside(int T, int E) { return E <= 256 && (T <= 16 || (T <= 32 && E <= 32)); }
+
+// Slices of H: enough workgroups (8 tokens x a slice) to spread over the
+// chip, few enough for the router to add up.
+int gate_splits(int T, int H, int* slice) {
+  int want = 256 / ((T + kGateT - 1) / kGateT);
+  want = want < 8 ? 8 : want > 16 ? 16 : want;
+  int n = ((H + want - 1) / want + 15) / 16 * 16;
+  n = n < 64 ? 64 : n > kGateMaxSlice ? kGateMaxSlice : n;
+  *slice = n;
+  return (H + n - 1) / n;
+}
+
+// The gating linear's slices into part; returns their number.
+int gate_launch(const uint16_t* x, const float* w_gate, int T, int H, int E, float* part,
+                hipStream_t s) {
+  int slice;
+  const int nsplit = gate_splits(T, H, &slice);
+  const dim3 grid((T + kGateT - 1) / kGateT, nsplit, (E + 63) / 64), block(256);
+  // LDS: the slice's tokens, later the sums of 256/EL row groups x 8 tokens x EL experts
+  const size_t lds = (size_t)(slice > 256 ? slice : 256) * kGateT * sizeof(float);
+#define SMOE_GATE(EL) gate_partial_kernel<EL><<<grid, block, lds, s>>>(x, w_gate, T, H, E, slice, part)
+  if (E <= 8) SMOE_GATE(8);
+  else if (E <= 16) SMOE_GATE(16);
+  else if (E <= 32) SMOE_GATE(32);
+  else SMOE_GATE(64);
+#undef SMOE_GATE
+  return nsplit;
+}
+}  // namespace
+
+extern "C" int smoe_gate_fused_ok(int T, int H, int E, int K) {
+  return T > 0 && H > 0 && H % kLane == 0 && E > 0 && E <= kGateMaxE && K > 0 && K <= E && K <= 32 &&
+         dispatch_small(T, K) && (long long)T * H * E <= kGateMaxWork;
+}
+
+extern "C" size_t smoe_route_dispatch_workspace_size(int T, int H, int E, int K) {
+  const size_t sort = smoe_route_sort_workspace_size(T, K, E);
+  if (!sort || !smoe_gate_fused_ok(T, H, E, K)) return sort;
+  int slice;
+  const size_t parts = kStatusBytes + (size_t)gate_splits(T, H, &slice) * T * E * sizeof(float);
+  return sort > parts ? sort : parts;
+}
+
+extern "C" int smoe_gate_logits(const uint16_t* x, const float* w_gate, int T, int H, int E, int K,
+                                float* logits, void* ws, size_t ws_bytes, void* stream) {
+  if (!smoe_gate_fused_ok(T, H, E, K)) return SMOE_EINVAL_DIM;
+  if (!w_gate || !logits) return SMOE_EINVAL_NULL;
+  if (((uintptr_t)w_gate | (uintptr_t)logits) & 3u) return SMOE_EINVAL_PTRALIGN;
+  SMOE_CHECK_PTR(x);
+  if (!ws || ws_bytes < smoe_route_dispatch_workspace_size(T, H, E, K)) return SMOE_EINVAL_WORKSPACE;
+  if ((uintptr_t)ws & 15u) return SMOE_EINVAL_PTRALIGN;
+  hipStream_t s = (hipStream_t)stream;
+  float* part = (float*)((char*)ws + kStatusBytes);
+  const int nsplit = gate_launch(x, w_gate, T, H, E, part, s), n = T * E;
+  gate_sum_kernel<<<dim3((n + 511) / 512), dim3(256), 0, s>>>(part, nsplit, n, logits);
+  SMOE_RETURN_LAUNCH();
+}
+
+extern "C" int smoe_route_dispatch(const uint16_t* x, const float* logits, const float* w_gate,
+                                   const float* bias, int T, int H, int E, int K,
+                                   int32_t* topk_idx, float* topk_w, int32_t* row_map,
+                                   int32_t* inv_map, int32_t* counts, int32_t* offsets,
+                                   uint8_t* xq, float* xs, int scale_mode, void* ws,
+                                   size_t ws_bytes, void* stream) {
+  if (!logits && !w_gate) return SMOE_EINVAL_NULL;
+  if (H <= 0) return SMOE_EINVAL_DIM;
+  if (H % kLane) return SMOE_EINVAL_ALIGN128;
+  if (scale_mode != SMOE_SCALE_AMAX && scale_mode != SMOE_SCALE_POW2) return SMOE_EINVAL_MODE;
+  int st = check_router_args(logits ? logits : w_gate, bias, T, E, K, topk_idx, topk_w);
+  if (st) return st;
+  st = check_sort_args(T, K, E, row_map, inv_map, counts, offsets, ws, ws_bytes, kSegR);
+  if (st) return st;
+  SMOE_CHECK_PTR(x);
+  SMOE_CHECK_PTR(inv_map);
+  SMOE_CHECK_PTR(xq);
+  SMOE_CHECK_PTR(xs);
+  if (!logits && (!smoe_gate_fused_ok(T, H, E, K) ||
+                  ws_bytes < smoe_route_dispatch_workspace_size(T, H, E, K)))
+    return smoe_gate_fused_ok(T, H, E, K) ? SMOE_EINVAL_WORKSPACE : SMOE_EINVAL_DIM;
+  hipStream_t s = (hipStream_t)stream;
+  if (!dispatch_small(T, K)) {
+    st = smoe_route_topk_sort(logits, bias, T, E, K, topk_idx, topk_w, row_map, inv_map, counts,
+                              offsets, ws, ws_bytes, stream);
+    return st ? st : smoe_permute_quant_ex(x, inv_map, T, H, K, xq, xs, scale_mode, stream);
+  }
+  int nsplit = 1;
+  const bool parts = !logits;
+  if (parts) {
+    float* part = (float*)((char*)ws + kStatusBytes);
+    nsplit = gate_launch(x, w_gate, T, H, E, part, s);
+    logits = part;
+  }
+  const bool inside = route_inside(T, E);
+  if (!inside && parts) {
+#define SMOE_ROUTER_P(NV) \
+  router_topk_kernel<16, NV, true><<<dim3((T + 15) / 16), dim3(256), 0, s>>>(logits, bias, T, E, K, topk_idx, topk_w, nsplit)
+    if (E <= 16) SMOE_ROUTER_P(1);
+    else if (E <= 32) SMOE_ROUTER_P(2);
+    else if (E <= 64) SMOE_ROUTER_P(4);
+    else if (E <= 128) SMOE_ROUTER_P(8);
+    else SMOE_ROUTER_P(16);
+#undef SMOE_ROUTER_P
+  } else if (!inside) {
+    st = smoe_router_topk(logits, bias, T, E, K, topk_idx, topk_w, stream);
+    if (st) return st;
+  }
+  const size_t lds = (size_t)(2 * E + (inside ? T * K + (parts ? T * E : 0) : 0)) * sizeof(int32_t);
+#define SMOE_DS(LPT, NV, RT, PT, P2)                                                              \
+  dispatch_small_kernel<LPT, NV, RT, PT, P2><<<dim3(T), dim3(256), lds, s>>>(                     \
+      logits, nsplit, bias, x, T, E, K, H, topk_idx, topk_w, row_map, inv_map, counts, offsets,   \
+      (int32_t*)ws, xq, xs)
+  const bool p2 = scale_mode == SMOE_SCALE_POW2;
+  if (!inside) {
+    if (p2) SMOE_DS(16, 1, false, false, true);
+    else SMOE_DS(16, 1, false, false, false);
+  } else {
+#define SMOE_DSR(LPT, NV)                          \
+  do {                                             \
+    if (parts) { if (p2) SMOE_DS(LPT, NV, true, true, true); else SMOE_DS(LPT, NV, true, true, false); }     \
+    else { if (p2) SMOE_DS(LPT, NV, true, false, true); else SMOE_DS(LPT, NV, true, false, false); }         \
+  } while (0)
+    if (E <= 16) SMOE_DSR(16, 1);
+    else if (E <= 32) SMOE_DSR(16, 2);
+    else if (E <= 64) SMOE_DSR(16, 4);
+    else if (E <= 128) SMOE_DSR(16, 8);
+    else SMOE_DSR(16, 16);
+#undef SMOE_DSR
+  }
+#undef SMOE_DS
   SMOE_RETURN_LAUNCH();
 }
 

@@ -28,6 +28,11 @@ SIGNATURES = {
     "smoe_route_sort_noalloc": (c_int, [P, c_int, c_int, c_int, P, P, P, P, P]),
     "smoe_route_topk_sort": (c_int, [P, P, c_int, c_int, c_int, P, P, P, P, P, P, P, c_size_t,
                                      P]),
+    "smoe_gate_fused_ok": (c_int, [c_int, c_int, c_int, c_int]),
+    "smoe_route_dispatch_workspace_size": (c_size_t, [c_int, c_int, c_int, c_int]),
+    "smoe_gate_logits": (c_int, [P, P, c_int, c_int, c_int, c_int, P, P, c_size_t, P]),
+    "smoe_route_dispatch": (c_int, [P, P, P, P, c_int, c_int, c_int, c_int, P, P, P, P, P, P, P, P,
+                                    c_int, P, c_size_t, P]),
     "smoe_permute_quant": (c_int, [P, P, c_int, c_int, c_int, P, P, P]),
     "smoe_permute_quant_ex": (c_int, [P, P, c_int, c_int, c_int, P, P, c_int, P]),
     "smoe_dispatch_quant": (c_int, [P, P, c_int, c_int, c_int, c_int, P, P, P, P, P, P, P,

@@ -77,6 +77,23 @@ class _SimpleMoEFunction(torch.autograd.Function):
         return g["dx"].to(ctx.dtypes[0]), g["dlogits"], grads[0], grads[1], None
 
 
+class _GateLinear(torch.autograd.Function):
+    """x.float() @ w_gate of a small batch by the layer's own kernel; the
+    backward is that product's."""
+
+    @staticmethod
+    def forward(ctx, x, w_gate, top_k):
+        ctx.save_for_backward(x, w_gate)
+        return ops.gate_logits(x.detach().contiguous(), w_gate.detach(), top_k)
+
+    @staticmethod
+    def backward(ctx, dlogits):
+        x, w_gate = ctx.saved_tensors
+        dx = (dlogits @ w_gate.t()).to(x.dtype) if ctx.needs_input_grad[0] else None
+        dw = x.float().t() @ dlogits if ctx.needs_input_grad[1] else None
+        return dx, dw, None
+
+
 class SimpleMoE(nn.Module):
     """Dropless top-k MoE FFN with SwiGLU experts in blockwise fp8.
 
@@ -238,33 +255,52 @@ class SimpleMoE(nn.Module):
         if return_intermediates:
             with torch.no_grad():
                 if logits is None:
-                    logits = x.float() @ self.w_gate
+                    logits = self._gate_logits(x)
                     out, inter = self._forward_impl(x, logits, save=True)
                     inter["logits_from_gate"] = True
                     return out, inter
                 return self._forward_impl(x, logits, save=True)
         if logits is None:
-            logits = x.float() @ self.w_gate
+            if self._gate_fused(x) and not (torch.is_grad_enabled() and any(
+                    t.requires_grad for t in (x, self.w_gate, self.w1, self.w2))):
+                return self._forward_impl(x, None, save=False)
+            logits = self._gate_logits(x)
         params = (x, logits, self.w1, self.w2)
         if torch.is_grad_enabled() and any(t.requires_grad for t in params):
             return _SimpleMoEFunction.apply(x, logits, self.w1, self.w2, self)
         with torch.no_grad():
             return self._forward_impl(x, logits, save=False)
 
+    def _gate_fused(self, x) -> bool:
+        """Whether the layer's own kernel runs the gating linear: a small batch
+        of plain bf16 tokens (an fp32 x is not rounded first, and autocast has
+        its own rule for the product).  Inference then forms the logits inside
+        the dispatch; the sums are the same with and without autograd."""
+        wg = self.w_gate
+        return (x.dtype == torch.bfloat16 and x.dim() == 2 and x.shape[1] == wg.shape[0]
+                and wg.dtype == torch.float32 and wg.is_contiguous() and wg.device == x.device
+                and not torch.is_autocast_enabled() and x.device.type == "cuda"
+                and ops.gate_fused_ok(x.shape[0], x.shape[1], wg.shape[1], self.top_k))
+
+    def _gate_logits(self, x):
+        if self._gate_fused(x):
+            return _GateLinear.apply(x, self.w_gate, self.top_k)
+        return x.float() @ self.w_gate
+
     @torch.no_grad()
-    def _forward_impl(self, x: torch.Tensor, logits: torch.Tensor, save: bool):
+    def _forward_impl(self, x: torch.Tensor, logits: torch.Tensor | None, save: bool):
+        """``logits`` None: formed from w_gate in the dispatch (_gate_fused)."""
         x = x.detach().to(torch.bfloat16).contiguous()
-        logits = logits.detach().float().contiguous()
+        if logits is not None:
+            logits = logits.detach().float().contiguous()
         if x.shape[0] == 0:
             return self._empty_forward(x, logits, save)
         fp8 = self.fp8_weights()
         w1q, w1s, w2q, w2s = self._gemm
-        # router and expert sort in three launches (the sort's histogram is
-        # counted inside the router launch)
-        idx, w, row_map, inv_map, counts, offsets = ops.route_topk_sort(logits, self.top_k,
-                                                                        self.router_bias)
         rs, e8 = self._row_scale, self._pow2
-        xq, xs = ops.permute_quant_rows(x, inv_map, self.top_k, scale=rs)
+        # router, expert sort and dispatch
+        idx, w, row_map, inv_map, counts, offsets, xq, xs = ops.route_dispatch(
+            x, logits, self.top_k, self.router_bias, scale=rs, w_gate=self.w_gate.detach())
         if save:
             # the backward pass needs c1 and bf16 h, so fc1 and SwiGLU run
             # as two kernels here

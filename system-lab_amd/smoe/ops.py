@@ -129,7 +129,10 @@ def _dev_key(device) -> torch.device:
 
 
 def _sort_workspace(T: int, K: int, E: int, dev) -> torch.Tensor:
-    nbytes = int(_C.lib().smoe_route_sort_workspace_size(T, K, E))
+    return _status_workspace(int(_C.lib().smoe_route_sort_workspace_size(T, K, E)), dev)
+
+
+def _status_workspace(nbytes: int, dev) -> torch.Tensor:
     ws = torch.empty(nbytes, dtype=torch.uint8, device=dev)
     # the status word of this call; check_route_status() reads it lazily
     _route_status[_dev_key(dev)] = ws[ROUTE_STATUS_OFFSET:ROUTE_STATUS_OFFSET + 4].view(torch.int32)
@@ -223,6 +226,61 @@ def route_topk_sort(logits: torch.Tensor, top_k: int, bias: torch.Tensor | None 
             _ptr(row_map), _ptr(inv_map), _ptr(counts), _ptr(offsets), _ptr(ws), ws.numel(),
             _stream())
     return idx, w, row_map, inv_map, counts, offsets
+
+
+def route_dispatch(x: torch.Tensor, logits: torch.Tensor | None, top_k: int,
+                   bias: torch.Tensor | None = None, scale: str = "amax",
+                   w_gate: torch.Tensor | None = None):
+    """``route_topk_sort`` then ``permute_quant_rows``, byte for byte, with
+    fewer launches for small batches.  -> (topk_idx, topk_w, row_map, inv_map,
+    counts, offsets, xq, xs).  With ``logits`` None they are x @ ``w_gate``
+    [H,E] in fp32 (where ``gate_fused_ok`` accepts the batch)."""
+    mode = _scale(scale)
+    _check(x, "x", (torch.bfloat16,), 2)
+    T, H = x.shape
+    gate = logits if logits is not None else w_gate
+    _check(gate, "logits" if logits is not None else "w_gate", (torch.float32,), 2)
+    E = gate.shape[1]
+    if gate.shape[0] != (T if logits is not None else H):
+        raise ValueError("logits must be [T, E] and w_gate [H, E] for x [T, H]")
+    if bias is not None:
+        _check(bias, "bias", (torch.float32,), 1)
+        if bias.numel() != E:
+            raise ValueError("bias must have E entries")
+    dev, R = x.device, T * top_k
+    i32 = dict(dtype=torch.int32, device=dev)
+    idx = torch.empty((T, top_k), **i32)
+    w = torch.empty((T, top_k), dtype=torch.float32, device=dev)
+    row_map, inv_map = torch.empty(R, **i32), torch.empty(R, **i32)
+    counts, offsets = torch.empty(E, **i32), torch.empty(E + 1, **i32)
+    xq = torch.empty((R, pad128(H)), dtype=FP8, device=dev)
+    xs = torch.empty((R, nblocks(H)), dtype=torch.float32, device=dev)
+    ws = _status_workspace(int(_C.lib().smoe_route_dispatch_workspace_size(T, H, E, top_k)), dev)
+    _C.call("smoe_route_dispatch", _ptr(x), _ptr(logits), _ptr(w_gate), _ptr(bias), T, H, E, top_k,
+            _ptr(idx), _ptr(w), _ptr(row_map), _ptr(inv_map), _ptr(counts), _ptr(offsets), _ptr(xq),
+            _ptr(xs), mode, _ptr(ws), ws.numel(), _stream())
+    return idx, w, row_map, inv_map, counts, offsets, xq, xs
+
+
+def gate_logits(x: torch.Tensor, w_gate: torch.Tensor, top_k: int) -> torch.Tensor:
+    """x [T,H] bf16 @ w_gate [H,E] f32 -> [T,E] f32, the logits
+    ``route_dispatch`` forms for the same batch (where ``gate_fused_ok``)."""
+    _check(x, "x", (torch.bfloat16,), 2)
+    _check(w_gate, "w_gate", (torch.float32,), 2)
+    (T, H), E = x.shape, w_gate.shape[1]
+    if w_gate.shape[0] != H:
+        raise ValueError("w_gate must be [H, E] for x [T, H]")
+    logits = torch.empty((T, E), dtype=torch.float32, device=x.device)
+    ws = torch.empty(int(_C.lib().smoe_route_dispatch_workspace_size(T, H, E, top_k)), dtype=torch.uint8,
+                     device=x.device)
+    _C.call("smoe_gate_logits", _ptr(x), _ptr(w_gate), T, H, E, top_k, _ptr(logits), _ptr(ws), ws.numel(),
+            _stream())
+    return logits
+
+
+def gate_fused_ok(T: int, H: int, E: int, top_k: int) -> bool:
+    """Whether ``route_dispatch`` forms the logits of such a batch itself."""
+    return bool(_C.lib().smoe_gate_fused_ok(T, H, E, top_k))
 
 
 # ---------------------------------------------------------------- dispatch
