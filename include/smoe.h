@@ -618,6 +618,86 @@ int smoe_combine_bwd_quant_cols(const uint16_t* dout, const int32_t* row_map, co
                                 uint8_t* dyTq, float* dyTs, int32_t* pad, int col_scale,
                                 void* stream);
 
+/*
+ * The whole expert layer in one call: the launches of smoe_route_dispatch, the
+ * two grouped GEMMs with SwiGLU + requantisation, and smoe_unpermute_combine,
+ * in order on the stream.  Shapes and buffers are those of the entry points
+ * it runs; w1 [E,2I,Hp], w2 [E,H,Ip] fp8 with their block scales, packed
+ * (smoe_pack_weight_fp8) where flags says so.  With scratch
+ * (smoe_layer_forward_scratch_size bytes) the intermediates live there and
+ * SwiGLU runs in the fc1 epilogue where that form exists (inference); with
+ * scratch NULL they are written to the caller's buffers topk_idx .. y for
+ * smoe_layer_backward.  logits NULL: formed from w_gate (smoe_gate_fused_ok).
+ * Replaces MoELayer.forward (moe/MoE_detailed_computation_dataflow.md:295-317).
+ */
+#define SMOE_LAYER_W1_PACKED 1
+#define SMOE_LAYER_W2_PACKED 2
+#define SMOE_LAYER_POW2 4      /* every row and weight scale a power of two */
+#define SMOE_LAYER_COL_POW2 8  /* backward: power-of-two column scales      */
+#define SMOE_LAYER_NO_JOIN 16  /* backward: the caller makes the stream wait */
+
+typedef struct {
+  int T, H, I, E, K, flags;
+  const uint16_t* x;
+  const float *logits, *w_gate, *bias;
+  const uint8_t* w1;
+  const float* w1s;
+  const uint8_t* w2;
+  const float* w2s;
+  uint16_t* out;
+  void* ws; /* smoe_route_dispatch_workspace_size bytes, status word first */
+  size_t ws_bytes;
+  void* scratch;
+  size_t scratch_bytes;
+  int32_t* topk_idx;
+  float* topk_w;
+  int32_t *row_map, *inv_map, *counts, *offsets;
+  uint8_t* xq;
+  float* xs;
+  uint16_t* c1;
+  uint8_t* hq;
+  float* hs;
+  uint16_t *h, *y;
+} smoe_layer_fwd;
+
+size_t smoe_layer_forward_scratch_size(int T, int H, int I, int E, int K, int flags);
+int smoe_layer_forward(const smoe_layer_fwd* args, void* stream);
+
+/*
+ * Its backward: combine backward, both dgrads, SwiGLU backward and the
+ * router's on the stream, the column quantisers and both wgrads on
+ * side_stream (which first waits for the stream, and which the stream waits
+ * for at the end, unless SMOE_LAYER_NO_JOIN leaves that to the caller).  w1t, w2t are the transposed weights (packed where flags
+ * says so), wgrad*_mode the SMOE_WGRAD_* modes of dw1, dw2.  Both streams use
+ * scratch (smoe_layer_backward_scratch_size bytes), which belongs to the
+ * stream: it is free again once the stream has waited for side_stream.
+ * Replaces the backward chain (moe/MoE_detailed_computation_dataflow.md:209-226).
+ */
+typedef struct {
+  int T, H, I, E, K, flags, wgrad1_mode, wgrad2_mode;
+  const uint16_t *dout, *x;
+  const float* logits;
+  const int32_t* topk_idx;
+  const float* topk_w;
+  const int32_t *row_map, *inv_map, *offsets;
+  const uint16_t *c1, *h, *y;
+  const uint8_t* w1t;
+  const float* w1ts;
+  const uint8_t* w2t;
+  const float* w2ts;
+  uint16_t* dx;
+  void *dw1, *dw2;
+  float *dtopk_w, *dlogits;
+  uint8_t* dyq;
+  float* dys;
+  uint16_t *dh, *dxs;
+  void* scratch;
+  size_t scratch_bytes;
+} smoe_layer_bwd;
+
+size_t smoe_layer_backward_scratch_size(int T, int H, int I, int E, int K);
+int smoe_layer_backward(const smoe_layer_bwd* args, void* stream, void* side_stream);
+
 #ifdef __cplusplus
 }
 #endif

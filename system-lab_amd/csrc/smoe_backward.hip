@@ -2,7 +2,7 @@
 // layer on gfx950: blockwise fp8 weight transpose (dgrad operands), 128x1
 // column quantisation into transposed, expert-segment-aligned layout (wgrad
 // operands), SwiGLU backward and combine backward.
-#include "smoe_common.h"
+#include "smoe_layer.h"
 
 namespace smoe {
 
@@ -547,10 +547,7 @@ extern "C" int smoe_quant_cols_ld(int R, int E) {
   return ld > 0x7fffffffLL ? 0 : (int)ld;
 }
 
-extern "C" int smoe_quant_cols_128x1(const uint16_t* x, const int32_t* gather, int gather_div,
-                                     int R, int C, const int32_t* offsets, int E, int ld,
-                                     uint8_t* xTq, float* xTs, int32_t* pad, int col_scale,
-                                     void* stream) {
+int smoe::quant_cols_128x1(const uint16_t* x, const int32_t* gather, int gather_div, int R, int C, const int32_t* offsets, int E, int ld, uint8_t* xTq, float* xTs, int32_t* pad, bool make_pad, int col_scale, void* stream) {
   if (R <= 0 || C <= 0) return SMOE_EINVAL_DIM;
   if (col_scale != SMOE_COLSCALE_FP32 && col_scale != SMOE_COLSCALE_POW2) return SMOE_EINVAL_MODE;
   if (gather && gather_div <= 0) return SMOE_EINVAL_DIM;
@@ -564,7 +561,7 @@ extern "C" int smoe_quant_cols_128x1(const uint16_t* x, const int32_t* gather, i
   if (!offsets || !xTs || !pad) return SMOE_EINVAL_NULL;
   if (((uintptr_t)offsets | (uintptr_t)xTs | (uintptr_t)pad) & 3u) return SMOE_EINVAL_PTRALIGN;
   hipStream_t s = (hipStream_t)stream;
-  pad_offsets_kernel<<<1, 1024, 0, s>>>(offsets, E, pad);
+  if (make_pad) pad_offsets_launch(offsets, E, pad, s);
   // column slabs vary fastest, so the workgroups in flight read whole rows
 #define SMOE_QC(P2)                                                                            \
   quant_cols_kernel<false, false, P2><<<dim3((C + kQcCols - 1) / kQcCols, ld / kGroup), dim3(256), 0, s>>>( \
@@ -576,9 +573,7 @@ extern "C" int smoe_quant_cols_128x1(const uint16_t* x, const int32_t* gather, i
   SMOE_RETURN_LAUNCH();
 }
 
-extern "C" int smoe_quant_rows_cols(const uint16_t* x, int R, int C, const int32_t* offsets, int E,
-                                    int ld, uint8_t* xq, float* xs, uint8_t* xTq, float* xTs,
-                                    int32_t* pad, int col_scale, void* stream) {
+int smoe::quant_rows_cols(const uint16_t* x, int R, int C, const int32_t* offsets, int E, int ld, uint8_t* xq, float* xs, uint8_t* xTq, float* xTs, int32_t* pad, bool make_pad, int col_scale, void* stream) {
   if (R <= 0 || C <= 0) return SMOE_EINVAL_DIM;
   if (col_scale & ~(SMOE_COLSCALE_POW2 | SMOE_ROWSCALE_POW2)) return SMOE_EINVAL_MODE;
   const bool cp2 = col_scale & SMOE_COLSCALE_POW2, rp2 = col_scale & SMOE_ROWSCALE_POW2;
@@ -594,7 +589,7 @@ extern "C" int smoe_quant_rows_cols(const uint16_t* x, int R, int C, const int32
   if (!xq) return SMOE_EINVAL_NULL;
   if ((uintptr_t)xq & 7u) return SMOE_EINVAL_PTRALIGN;
   hipStream_t s = (hipStream_t)stream;
-  pad_offsets_kernel<<<1, 1024, 0, s>>>(offsets, E, pad);
+  if (make_pad) pad_offsets_launch(offsets, E, pad, s);
 #define SMOE_QRC(P2, RP2)                                                                      \
   quant_cols_kernel<true, false, P2, RP2><<<dim3((C + kQcCols - 1) / kQcCols, ld / kGroup), dim3(256), 0, s>>>( \
       x, nullptr, 1, nullptr, R, C, offsets, pad, E, ld, xTq, xTs, xq, xs, nullptr, nullptr, nullptr)
@@ -604,10 +599,7 @@ extern "C" int smoe_quant_rows_cols(const uint16_t* x, int R, int C, const int32
   SMOE_RETURN_LAUNCH();
 }
 
-extern "C" int smoe_swiglu_bwd_quant(const uint16_t* c1, const uint16_t* dh, int R, int I,
-                                     const int32_t* offsets, int E, int ld, uint8_t* dcq,
-                                     float* dcs, uint8_t* dcTq, float* dcTs, int32_t* pad,
-                                     uint16_t* dc1, int col_scale, void* stream) {
+int smoe::swiglu_bwd_quant(const uint16_t* c1, const uint16_t* dh, int R, int I, const int32_t* offsets, int E, int ld, uint8_t* dcq, float* dcs, uint8_t* dcTq, float* dcTs, int32_t* pad, bool make_pad, uint16_t* dc1, int col_scale, void* stream) {
   if (R <= 0 || I <= 0) return SMOE_EINVAL_DIM;
   if (col_scale & ~(SMOE_COLSCALE_POW2 | SMOE_ROWSCALE_POW2)) return SMOE_EINVAL_MODE;
   const bool cp2 = col_scale & SMOE_COLSCALE_POW2, rp2 = col_scale & SMOE_ROWSCALE_POW2;
@@ -625,7 +617,7 @@ extern "C" int smoe_swiglu_bwd_quant(const uint16_t* c1, const uint16_t* dh, int
   if (dc1 && ((uintptr_t)dc1 & 15u)) return SMOE_EINVAL_PTRALIGN;
   const int C = 2 * I;
   hipStream_t s = (hipStream_t)stream;
-  pad_offsets_kernel<<<1, 1024, 0, s>>>(offsets, E, pad);
+  if (make_pad) pad_offsets_launch(offsets, E, pad, s);
   // one workgroup per 128-column block of both halves (dg and du)
 #define SMOE_SBQ(P2, RP2)                                                          \
   quant_cols_kernel<true, true, P2, RP2><<<dim3(I / kQcCols, ld / kGroup), dim3(256), 0, s>>>( \
@@ -671,6 +663,10 @@ extern "C" int smoe_unpermute_combine_bwd(const uint16_t* dout, const uint16_t* 
   SMOE_RETURN_LAUNCH();
 }
 
+void smoe::pad_offsets_launch(const int32_t* offsets, int E, int32_t* pad, hipStream_t s) {
+  pad_offsets_kernel<<<1, 1024, 0, s>>>(offsets, E, pad);
+}
+
 namespace {
 // The 128x1 columns of dy: row r of dy is rebuilt as bf16(w[p] * dout[p / K])
 // with p = row_map[r].
@@ -688,13 +684,7 @@ void combine_bwd_cols_launch(const uint16_t* dout, const int32_t* row_map, const
 }
 }  // namespace
 
-extern "C" int smoe_unpermute_combine_bwd_quant(const uint16_t* dout, const uint16_t* y,
-                                                const int32_t* inv_map, const int32_t* row_map,
-                                                const float* w, int T, int K, int H,
-                                                const int32_t* offsets, int E, int ld,
-                                                uint8_t* dyq, float* dys, uint8_t* dyTq,
-                                                float* dyTs, int32_t* pad, float* dw,
-                                                int col_scale, void* stream) {
+int smoe::combine_bwd_quant(const uint16_t* dout, const uint16_t* y, const int32_t* inv_map, const int32_t* row_map, const float* w, int T, int K, int H, const int32_t* offsets, int E, int ld, uint8_t* dyq, float* dys, uint8_t* dyTq, float* dyTs, int32_t* pad, bool make_pad, float* dw, int col_scale, void* stream) {
   if (T <= 0 || H <= 0) return SMOE_EINVAL_DIM;
   if (col_scale & ~(SMOE_COLSCALE_POW2 | SMOE_ROWSCALE_POW2)) return SMOE_EINVAL_MODE;
   const bool cp2 = col_scale & SMOE_COLSCALE_POW2, rp2 = col_scale & SMOE_ROWSCALE_POW2;
@@ -733,16 +723,12 @@ extern "C" int smoe_unpermute_combine_bwd_quant(const uint16_t* dout, const uint
     else SMOE_CBB(32, false);
   }
 #undef SMOE_CBB
-  pad_offsets_kernel<<<1, 1024, 0, s>>>(offsets, E, pad);
+  if (make_pad) pad_offsets_launch(offsets, E, pad, s);
   if (cols) combine_bwd_cols_launch(dout, row_map, w, K, R, H, offsets, E, ld, dyTq, dyTs, pad, cp2, s);
   SMOE_RETURN_LAUNCH();
 }
 
-extern "C" int smoe_combine_bwd_quant_cols(const uint16_t* dout, const int32_t* row_map,
-                                           const float* w, int T, int K, int H,
-                                           const int32_t* offsets, int E, int ld, uint8_t* dyTq,
-                                           float* dyTs, int32_t* pad, int col_scale,
-                                           void* stream) {
+int smoe::combine_bwd_quant_cols(const uint16_t* dout, const int32_t* row_map, const float* w, int T, int K, int H, const int32_t* offsets, int E, int ld, uint8_t* dyTq, float* dyTs, int32_t* pad, bool make_pad, int col_scale, void* stream) {
   if (T <= 0 || H <= 0) return SMOE_EINVAL_DIM;
   if (col_scale & ~SMOE_COLSCALE_POW2) return SMOE_EINVAL_MODE;
   if (H % kLane) return SMOE_EINVAL_ALIGN128;
@@ -759,8 +745,48 @@ extern "C" int smoe_combine_bwd_quant_cols(const uint16_t* dout, const int32_t* 
        (uintptr_t)pad) & 3u)
     return SMOE_EINVAL_PTRALIGN;
   hipStream_t s = (hipStream_t)stream;
-  pad_offsets_kernel<<<1, 1024, 0, s>>>(offsets, E, pad);
+  if (make_pad) pad_offsets_launch(offsets, E, pad, s);
   combine_bwd_cols_launch(dout, row_map, w, K, R, H, offsets, E, ld, dyTq, dyTs, pad,
                           col_scale & SMOE_COLSCALE_POW2, s);
   SMOE_RETURN_LAUNCH();
+}
+
+// ------------------------------------------- the entry points of these
+extern "C" int smoe_quant_cols_128x1(const uint16_t* x, const int32_t* gather, int gather_div, int
+                                     R, int C, const int32_t* offsets, int E, int ld, uint8_t* xTq,
+                                     float* xTs, int32_t* pad, int col_scale, void* stream) {
+  return quant_cols_128x1(x, gather, gather_div, R, C, offsets, E, ld, xTq, xTs, pad, true,
+      col_scale, stream);
+}
+
+extern "C" int smoe_quant_rows_cols(const uint16_t* x, int R, int C, const int32_t* offsets, int E,
+                                    int ld, uint8_t* xq, float* xs, uint8_t* xTq, float* xTs,
+                                    int32_t* pad, int col_scale, void* stream) {
+  return quant_rows_cols(x, R, C, offsets, E, ld, xq, xs, xTq, xTs, pad, true, col_scale, stream);
+}
+
+extern "C" int smoe_swiglu_bwd_quant(const uint16_t* c1, const uint16_t* dh, int R, int I, const
+                                     int32_t* offsets, int E, int ld, uint8_t* dcq, float* dcs,
+                                     uint8_t* dcTq, float* dcTs, int32_t* pad, uint16_t* dc1, int
+                                     col_scale, void* stream) {
+  return swiglu_bwd_quant(c1, dh, R, I, offsets, E, ld, dcq, dcs, dcTq, dcTs, pad, true, dc1,
+      col_scale, stream);
+}
+
+extern "C" int smoe_unpermute_combine_bwd_quant(const uint16_t* dout, const uint16_t* y, const
+                                                int32_t* inv_map, const int32_t* row_map, const
+                                                float* w, int T, int K, int H, const int32_t*
+                                                offsets, int E, int ld, uint8_t* dyq, float* dys,
+                                                uint8_t* dyTq, float* dyTs, int32_t* pad, float* dw,
+                                                int col_scale, void* stream) {
+  return combine_bwd_quant(dout, y, inv_map, row_map, w, T, K, H, offsets, E, ld, dyq, dys, dyTq,
+      dyTs, pad, true, dw, col_scale, stream);
+}
+
+extern "C" int smoe_combine_bwd_quant_cols(const uint16_t* dout, const int32_t* row_map, const
+                                           float* w, int T, int K, int H, const int32_t* offsets,
+                                           int E, int ld, uint8_t* dyTq, float* dyTs, int32_t* pad,
+                                           int col_scale, void* stream) {
+  return combine_bwd_quant_cols(dout, row_map, w, T, K, H, offsets, E, ld, dyTq, dyTs, pad, true,
+      col_scale, stream);
 }

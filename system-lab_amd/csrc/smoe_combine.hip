@@ -5,7 +5,7 @@
 // its token (K 128-bit loads in flight), accumulates w[t,k] * y in fp32 in
 // k order with separately rounded multiply and add, and writes the bf16
 // (round-to-nearest-even) result with one 128-bit non-temporal store.
-#include "smoe_common.h"
+#include "smoe_layer.h"
 
 namespace smoe {
 
@@ -39,7 +39,7 @@ __global__ __launch_bounds__(256) void combine_kernel(const uint16_t* __restrict
   for (int k = 0; k < kMaxK; ++k) {
     if (k < K) {
       r[k] = inv_map[(size_t)t * K + k];
-      wk[k] = w[(size_t)t * K + k];
+      wk[k] = w ? w[(size_t)t * K + k] : 1.0f;  // no weights: a plain sum
       if ((unsigned)r[k] >= (unsigned)R) {  // malformed map: contribute nothing
         r[k] = 0;
         wk[k] = 0.0f;
@@ -93,15 +93,15 @@ constexpr bool kCombineNT = true;
 
 using namespace smoe;
 
-extern "C" int smoe_unpermute_combine(const uint16_t* y, const int32_t* inv_map, const float* w,
-                                      int T, int K, int H, uint16_t* out, void* stream) {
+int smoe::combine_launch(const uint16_t* y, const int32_t* inv_map, const float* w, int T, int K,
+                         int H, uint16_t* out, void* stream) {
   if (T <= 0 || H <= 0) return SMOE_EINVAL_DIM;
   if (H % kLane) return SMOE_EINVAL_ALIGN128;  // whole 16-byte lane pieces
   if (K <= 0 || K > 32) return SMOE_EINVAL_TOPK;
   if ((long long)T * K > 0x7fffffffLL) return SMOE_EINVAL_DIM;
   SMOE_CHECK_PTR(y);
   SMOE_CHECK_PTR(out);
-  if (!inv_map || !w) return SMOE_EINVAL_NULL;
+  if (!inv_map) return SMOE_EINVAL_NULL;
   if (((uintptr_t)inv_map | (uintptr_t)w) & 3u) return SMOE_EINVAL_PTRALIGN;
   const dim3 grid((T + 3) / 4), block(256);
   hipStream_t s = (hipStream_t)stream;
@@ -114,4 +114,9 @@ extern "C" int smoe_unpermute_combine(const uint16_t* y, const int32_t* inv_map,
   else SMOE_CB(32);
 #undef SMOE_CB
   SMOE_RETURN_LAUNCH();
+}
+
+extern "C" int smoe_unpermute_combine(const uint16_t* y, const int32_t* inv_map, const float* w,
+                                      int T, int K, int H, uint16_t* out, void* stream) {
+  return w ? combine_launch(y, inv_map, w, T, K, H, out, stream) : SMOE_EINVAL_NULL;
 }

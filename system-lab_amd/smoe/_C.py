@@ -75,9 +75,31 @@ SIGNATURES = {
     "smoe_unpermute_combine_bwd": (c_int, [P, P, P, P, c_int, c_int, c_int, P, P, P]),
     "smoe_unpermute_combine_bwd_quant": (c_int, [P, P, P, P, P, c_int, c_int, c_int, P, c_int,
                                                  c_int, P, P, P, P, P, P, c_int, P]),
+    "smoe_layer_forward_scratch_size": (c_size_t, [c_int] * 6),
+    "smoe_layer_forward": (c_int, [P, P]),
+    "smoe_layer_backward_scratch_size": (c_size_t, [c_int] * 5),
+    "smoe_layer_backward": (c_int, [P, P, P]),
     "smoe_combine_bwd_quant_cols": (c_int, [P, P, P, c_int, c_int, c_int, P, c_int, c_int, P, P,
                                             P, c_int, P]),
 }
+
+
+class LayerFwd(ctypes.Structure):
+    """smoe_layer_fwd"""
+    _fields_ = ([(n, c_int) for n in ("T", "H", "I", "E", "K", "flags")]
+                + [(n, P) for n in ("x", "logits", "w_gate", "bias", "w1", "w1s", "w2", "w2s", "out", "ws")]
+                + [("ws_bytes", c_size_t), ("scratch", P), ("scratch_bytes", c_size_t)]
+                + [(n, P) for n in ("topk_idx", "topk_w", "row_map", "inv_map", "counts", "offsets", "xq",
+                                    "xs", "c1", "hq", "hs", "h", "y")])
+
+
+class LayerBwd(ctypes.Structure):
+    """smoe_layer_bwd"""
+    _fields_ = ([(n, c_int) for n in ("T", "H", "I", "E", "K", "flags", "wgrad1_mode", "wgrad2_mode")]
+                + [(n, P) for n in ("dout", "x", "logits", "topk_idx", "topk_w", "row_map", "inv_map",
+                                    "offsets", "c1", "h", "y", "w1t", "w1ts", "w2t", "w2ts", "dx", "dw1",
+                                    "dw2", "dtopk_w", "dlogits", "dyq", "dys", "dh", "dxs", "scratch")]
+                + [("scratch_bytes", c_size_t)])
 
 
 # libsmoe_probe.so: the benchmark's HBM traffic-mix probe, kept out of the
@@ -124,6 +146,9 @@ def call(name: str, *args) -> None:
     st = getattr(lib(), name)(*args)
     if st != 0:
         raise SmoeError(name, st, lib().smoe_strerror(st).decode())
+
+
+SMOE_LAYER_W1_PACKED, SMOE_LAYER_W2_PACKED, SMOE_LAYER_POW2, SMOE_LAYER_COL_POW2, SMOE_LAYER_NO_JOIN = 1, 2, 4, 8, 16
 
 
 _probe = None

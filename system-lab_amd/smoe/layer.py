@@ -9,10 +9,12 @@ forward is stream-ordered with no host synchronisation.
 """
 from __future__ import annotations
 
+import ctypes
+
 import torch
 from torch import nn
 
-from . import ops
+from . import _C, ops
 
 
 # Optimizer steps seen in this process.  Megatron-style optimizers write the
@@ -296,26 +298,58 @@ class SimpleMoE(nn.Module):
         if x.shape[0] == 0:
             return self._empty_forward(x, logits, save)
         fp8 = self.fp8_weights()
-        w1q, w1s, w2q, w2s = self._gemm
-        rs, e8 = self._row_scale, self._pow2
-        # router, expert sort and dispatch
-        idx, w, row_map, inv_map, counts, offsets, xq, xs = ops.route_dispatch(
-            x, logits, self.top_k, self.router_bias, scale=rs, w_gate=self.w_gate.detach())
+        w1, w1s, w2, w2s = self._gemm
+        H, I, E, K = self.hidden, self.intermediate, self.num_experts, self.top_k
+        ops._check(x, "x", (torch.bfloat16,), 2)
+        T, dev = x.shape[0], x.device
+        if x.shape[1] != H:
+            raise ValueError(f"x must be [T, {H}], got {tuple(x.shape)}")
+        gate = logits if logits is not None else self.w_gate.detach()
+        ops._check(gate, "logits", (torch.float32,), 2)
+        if tuple(gate.shape) != ((T if logits is not None else H), E):
+            raise ValueError(f"logits must be [{T}, {E}], got {tuple(gate.shape)}")
+        bias = self.router_bias
+        if bias is not None:
+            ops._check(bias, "router_bias", (torch.float32,), 1)
+            if bias.numel() != E:
+                raise ValueError("router_bias must have E entries")
+        if w1.device != dev:
+            raise ValueError(f"the weights are on {w1.device}, x on {dev}")
+        flags = self._layer_flags(w1, w2)
+        lib = _C.lib()
+        out = torch.empty((T, H), dtype=torch.bfloat16, device=dev)
+        ws = ops._status_workspace(lib.smoe_route_dispatch_workspace_size(T, H, E, K), dev)
+        a = _C.LayerFwd(T, H, I, E, K, flags, x.data_ptr(), None if logits is None else gate.data_ptr(),
+                        gate.data_ptr() if logits is None else None, None if bias is None else bias.data_ptr(),
+                        ops._gemm_ptr(w1), w1s.data_ptr(), ops._gemm_ptr(w2), w2s.data_ptr(), out.data_ptr(),
+                        ws.data_ptr(), ws.numel())
+        inter = None
         if save:
-            # the backward pass needs c1 and bf16 h, so fc1 and SwiGLU run
-            # as two kernels here
-            c1 = ops.grouped_gemm_fp8(xq, xs, w1q, w1s, offsets, e8m0=e8)
-            hq, hs, h = ops.swiglu_quant(c1, save_h=True, scale=rs)
+            # the intermediates of a later backward, which needs c1 and bf16
+            # h: fc1 and SwiGLU run as two kernels
+            R, new = T * K, lambda dt, *shape: torch.empty(shape, dtype=dt, device=dev)
+            inter = dict(x=x, logits=logits, topk_idx=new(torch.int32, T, K), topk_w=new(torch.float32, T, K),
+                         row_map=new(torch.int32, R), inv_map=new(torch.int32, R), counts=new(torch.int32, E),
+                         offsets=new(torch.int32, E + 1), xq=new(ops.FP8, R, ops.pad128(H)),
+                         xs=new(torch.float32, R, ops.nblocks(H)), c1=new(torch.bfloat16, R, 2 * I),
+                         hq=new(ops.FP8, R, ops.pad128(I)), hs=new(torch.float32, R, ops.nblocks(I)),
+                         h=new(torch.bfloat16, R, I), y=new(torch.bfloat16, R, H), fp8=fp8)
+            for k in ("topk_idx", "topk_w", "row_map", "inv_map", "counts", "offsets", "xq", "xs", "c1", "hq",
+                      "hs", "h", "y"):
+                setattr(a, k, inter[k].data_ptr())
         else:
-            # inference: SwiGLU + requantisation run in the fc1 epilogue
-            hq, hs = ops.grouped_gemm_fp8_swiglu(xq, xs, w1q, w1s, offsets, scale=rs)
-        y = ops.grouped_gemm_fp8(hq, hs, w2q, w2s, offsets, e8m0=e8)
-        out = ops.unpermute_combine(y, inv_map, w)
-        if save:
-            return out, dict(x=x, logits=logits, topk_idx=idx, topk_w=w, row_map=row_map,
-                             inv_map=inv_map, counts=counts, offsets=offsets, xq=xq, xs=xs,
-                             c1=c1, hq=hq, hs=hs, h=h, y=y, fp8=fp8)
-        return out
+            # inference: SwiGLU + requantisation run in the fc1 epilogue and
+            # the intermediates live in one buffer
+            nbytes = lib.smoe_layer_forward_scratch_size(T, H, I, E, K, flags)
+            buf = torch.empty(nbytes, dtype=torch.uint8, device=dev)
+            a.scratch, a.scratch_bytes = buf.data_ptr(), nbytes
+        _C.call("smoe_layer_forward", ctypes.byref(a), ops._stream())
+        return (out, inter) if save else out
+
+    def _layer_flags(self, w1, w2) -> int:
+        return ((_C.SMOE_LAYER_W1_PACKED if isinstance(w1, ops.PackedWeight) else 0)
+                | (_C.SMOE_LAYER_W2_PACKED if isinstance(w2, ops.PackedWeight) else 0)
+                | (_C.SMOE_LAYER_POW2 if self._pow2 else 0))
 
     def _empty_forward(self, x: torch.Tensor, logits: torch.Tensor, save: bool):
         """An empty batch (T = 0): no kernel runs (the C ABI rejects T = 0);
@@ -397,9 +431,20 @@ class SimpleMoE(nn.Module):
             if dw2_into is not None:
                 out["dw2"] = dw2_into
             return out
-        w1tq, w1ts, w2tq, w2ts = self.gemm_weights_t(inter.get("fp8"))
-        off, inv = inter["offsets"], inter["inv_map"]
-        K = self.top_k
+        w1t, w1ts, w2t, w2ts = self.gemm_weights_t(inter.get("fp8"))
+        K, T = self.top_k, inter["x"].shape[0]
+        R, dev = T * K, dout.device
+        dout = dout.contiguous()
+        i32, f32, bf16 = torch.int32, torch.float32, torch.bfloat16
+        for t, name, dt, shape in (
+                (dout, "dout", bf16, (T, H)), (inter["x"], "x", bf16, (T, H)), (inter["logits"], "logits", f32, (T, E)),
+                (inter["topk_idx"], "topk_idx", i32, (T, K)), (inter["topk_w"], "topk_w", f32, (T, K)),
+                (inter["row_map"], "row_map", i32, (R,)), (inter["inv_map"], "inv_map", i32, (R,)),
+                (inter["offsets"], "offsets", i32, (E + 1,)), (inter["c1"], "c1", bf16, (R, 2 * I)),
+                (inter["h"], "h", bf16, (R, I)), (inter["y"], "y", bf16, (R, H))):
+            ops._check(t, name, (dt,))
+            if tuple(t.shape) != shape:
+                raise ValueError(f"{name} must be {list(shape)}, got {list(t.shape)}")
         # The weight gradients are off the dx critical path.  They run on a
         # second stream (default priority), so that a wgrad tile writing its
         # fp32 output shares the chip with dgrad tiles that are MFMA-bound.
@@ -408,56 +453,40 @@ class SimpleMoE(nn.Module):
         main = torch.cuda.current_stream()
         side = self._side_stream(main.device)
         e8m0 = self.wgrad_recipe == "e8m0" or self._pow2
-        cs = "pow2" if e8m0 else "fp32"
-        rs, e8 = self._row_scale, self._pow2
-        ones = torch.ones_like(inter["topk_w"])
+        new = lambda dt, *shape: torch.empty(shape, dtype=dt, device=dev)
         # the returned weight gradients are allocated on the caller's stream,
         # so the caching allocator never hands their memory to side-stream
         # work while the caller still uses them
-        dw1 = dw1_into if dw1_into is not None else torch.empty((E, 2 * I, H), dtype=wgrad_dtype,
-                                                                device=dout.device)
-        dw2 = dw2_into if dw2_into is not None else torch.empty((E, H, I), dtype=wgrad_dtype,
-                                                                device=dout.device)
-        dout = dout.contiguous()
-        side.wait_stream(main)
-        with torch.cuda.stream(side):
-            # the wgrad activation operands depend on the forward only: h, and
-            # the sorted tokens x[row_map // K] gathered inside the quantiser
-            hTq, hTs, _, _ = ops.quant_cols(inter["h"], off, col_scale=cs)
-            xTq, xTs, _, _ = ops.quant_cols(inter["x"], off, gather=inter["row_map"], gather_div=K,
-                                            col_scale=cs)
-        # combine backward fused with dy's 1x128 row quantisation for the
-        # dgrad; the 128x1 columns for the wgrad (rebuilt from dout, not from
-        # the row pass) on the side stream; dy itself is never stored
-        with torch.cuda.stream(side):
-            dyTq, dyTs, pad, ld = ops.combine_bwd_quant_cols(dout, inter["row_map"],
-                                                             inter["topk_w"], off, col_scale=cs)
-            ops.grouped_gemm_fp8_wgrad(dyTq, dyTs, hTq, hTs, pad, ld, out=dw2,
-                                       accumulate=dw2_into is not None, e8m0=e8m0)
-        dyq, dys, _, _, _, _, dw = ops.unpermute_combine_bwd_quant(
-            dout, inter["y"], inv, inter["row_map"], inter["topk_w"], off, col_scale=cs,
-            row_scale=rs, cols=False)
-        dh = ops.grouped_gemm_fp8(dyq, dys, w2tq, w2ts, off, e8m0=e8)
-        # SwiGLU backward fused with both quantisations of dc1 (dc1 itself is
-        # never stored)
-        dcq, dcs, dcTq, dcTs, _, _ = ops.swiglu_bwd_quant(inter["c1"], dh, off, col_scale=cs,
-                                                          row_scale=rs)
-        side.wait_stream(main)
-        with torch.cuda.stream(side):
-            ops.grouped_gemm_fp8_wgrad(dcTq, dcTs, xTq, xTs, pad, ld, out=dw1,
-                                       accumulate=dw1_into is not None, e8m0=e8m0)
-        dxs = ops.grouped_gemm_fp8(dcq, dcs, w1tq, w1ts, off, e8m0=e8)
-        dx = ops.unpermute_combine(dxs, inv, ones)
-        # router: renormalisation + softmax backward into the logits
-        dlogits = ops.router_topk_bwd(inter["logits"], inter["topk_idx"], dw)
-        out = dict(dx=dx, dw1=dw1, dw2=dw2, dtopk_w=dw, dlogits=dlogits, dyq=dyq, dys=dys,
-                   dh=dh, dxs=dxs)
-        if inter.get("logits_from_gate"):
+        dw1 = dw1_into if dw1_into is not None else new(wgrad_dtype, E, 2 * I, H)
+        dw2 = dw2_into if dw2_into is not None else new(wgrad_dtype, E, H, I)
+        modes = [ops.WGRAD_MODES[(d.dtype, into is not None)] | (ops.WGRAD_E8M0 if e8m0 else 0)
+                 for d, into in ((dw1, dw1_into), (dw2, dw2_into))]
+        out = dict(dx=new(bf16, T, H), dw1=dw1, dw2=dw2, dtopk_w=new(f32, T, K), dlogits=new(f32, T, E),
+                   dyq=new(ops.FP8, R, ops.pad128(H)), dys=new(f32, R, ops.nblocks(H)), dh=new(bf16, R, I),
+                   dxs=new(bf16, R, H))
+        lib = _C.lib()
+        # both streams' scratch is the caller's stream's memory: that stream
+        # waits for the side stream before anything later can reuse it
+        nbytes = lib.smoe_layer_backward_scratch_size(T, H, I, E, K)
+        scratch = new(torch.uint8, nbytes)
+        flags = self._layer_flags(w1t, w2t) | (_C.SMOE_LAYER_COL_POW2 if e8m0 else 0)
+        gate = inter.get("logits_from_gate")
+        if gate:  # more work for this stream before it waits for the side stream
+            flags |= _C.SMOE_LAYER_NO_JOIN
+        a = _C.LayerBwd(T, H, I, E, K, flags, modes[0], modes[1], dout.data_ptr(),
+                        *(inter[k].data_ptr() for k in ("x", "logits", "topk_idx", "topk_w", "row_map",
+                                                        "inv_map", "offsets", "c1", "h", "y")),
+                        ops._gemm_ptr(w1t), w1ts.data_ptr(), ops._gemm_ptr(w2t), w2ts.data_ptr(),
+                        *(out[k].data_ptr() for k in ("dx", "dw1", "dw2", "dtopk_w", "dlogits", "dyq", "dys",
+                                                      "dh", "dxs")),
+                        scratch.data_ptr(), nbytes)
+        _C.call("smoe_layer_backward", ctypes.byref(a), main.cuda_stream, side.cuda_stream)
+        if gate:
             # logits = x @ w_gate in fp32: the gating linear's gradients
-            x32 = inter["x"].float()
-            out["dx"] = (dx.float() + dlogits @ self.w_gate.detach().t()).to(torch.bfloat16)
+            x32, dlogits = inter["x"].float(), out["dlogits"]
+            out["dx"] = (out["dx"].float() + dlogits @ self.w_gate.detach().t()).to(torch.bfloat16)
             out["dw_gate"] = x32.t() @ dlogits
-        main.wait_stream(side)
+            main.wait_stream(side)
         return out
 
     def _side_stream(self, device) -> torch.cuda.Stream:

@@ -430,6 +430,11 @@ def quantize_pack_weight(w: torch.Tensor, scale: str = "amax"):
     return wq, ws, PackedWeight(wp)
 
 
+def _gemm_ptr(w) -> int:
+    """Address of a weight in the form the GEMMs take it."""
+    return (w.data if isinstance(w, PackedWeight) else w).data_ptr()
+
+
 def _weight(wq, name):
     """(tensor, packed?) of a GEMM weight argument."""
     if isinstance(wq, PackedWeight):
