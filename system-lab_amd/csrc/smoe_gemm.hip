@@ -406,7 +406,7 @@ extern "C" int smoe_grouped_gemm_fp8(const uint8_t* a, const float* as, const ui
   SMOE_CHECK_PTR(c);
   if (!as || !bs || !offsets) return SMOE_EINVAL_NULL;
   if (((uintptr_t)as | (uintptr_t)bs | (uintptr_t)offsets) & 3u) return SMOE_EINVAL_PTRALIGN;
-  if (small_gemm_rows(SmallWeights::kPlain, E, R))
+  if (small_gemm_rows(SmallWeights::kPlain, false, false, E, R, N, Kdim))
     return small_gemm_launch(SmallWeights::kPlain, false, a, as, b, bs, offsets, E, R, N, Kdim, c,
                              nullptr, nullptr, (hipStream_t)stream);
   using C = GemmCfg;
@@ -446,7 +446,7 @@ extern "C" int smoe_grouped_gemm_fp8_swiglu(const uint8_t* a, const float* as, c
   if (((uintptr_t)as | (uintptr_t)w1s | (uintptr_t)offsets | (uintptr_t)hs) & 3u)
     return SMOE_EINVAL_PTRALIGN;
   const int N = 2 * I;
-  if (small_gemm_rows(SmallWeights::kPlain, E, R))
+  if (small_gemm_rows(SmallWeights::kPlain, false, true, E, R, 2 * I, Kdim))
     return small_gemm_launch(SmallWeights::kPlain, false, a, as, w1, w1s, offsets, E, R, N, Kdim,
                              c1, hq, hs, (hipStream_t)stream);
   using C = GemmCfg;

@@ -444,7 +444,7 @@ extern "C" int smoe_grouped_gemm_fp8_packed_e8m0(const uint8_t* a, const float* 
   const int st = e8m0_args(a, as, wp, ws, offsets, E, R, N, Kdim);
   if (st) return st;
   SMOE_CHECK_PTR(c);
-  if (small_gemm_rows(SmallWeights::kPacked, E, R))
+  if (small_gemm_rows(SmallWeights::kPacked, true, false, E, R, N, Kdim))
     return small_gemm_launch(SmallWeights::kPacked, true, a, as, wp, ws, offsets, E, R, N, Kdim, c,
                              nullptr, nullptr, (hipStream_t)stream);
   long long mt_bound;
@@ -469,7 +469,7 @@ extern "C" int smoe_grouped_gemm_fp8_packed_e8m0_swiglu(const uint8_t* a, const 
   if (c1 && ((uintptr_t)c1 & 15u)) return SMOE_EINVAL_PTRALIGN;
   if (!hs) return SMOE_EINVAL_NULL;
   if ((uintptr_t)hs & 3u) return SMOE_EINVAL_PTRALIGN;
-  if (small_gemm_rows(SmallWeights::kPacked, E, R))
+  if (small_gemm_rows(SmallWeights::kPacked, true, true, E, R, 2 * I, Kdim))
     return small_gemm_launch(SmallWeights::kPacked, true, a, as, w1p, w1s, offsets, E, R, 2 * I,
                              Kdim, c1, hq, hs, (hipStream_t)stream);
   long long mt_bound;

@@ -427,7 +427,7 @@ extern "C" int smoe_grouped_gemm_fp8_packed(const uint8_t* a, const float* as, c
   const int st = packed_args(a, as, wp, ws, offsets, E, R, N, Kdim);
   if (st) return st;
   SMOE_CHECK_PTR(c);
-  if (small_gemm_rows(SmallWeights::kPacked, E, R))
+  if (small_gemm_rows(SmallWeights::kPacked, false, false, E, R, N, Kdim))
     return small_gemm_launch(SmallWeights::kPacked, false, a, as, wp, ws, offsets, E, R, N, Kdim,
                              c, nullptr, nullptr, (hipStream_t)stream);
   long long mt_bound;
@@ -452,7 +452,7 @@ extern "C" int smoe_grouped_gemm_fp8_packed_swiglu(const uint8_t* a, const float
   if (c1 && ((uintptr_t)c1 & 15u)) return SMOE_EINVAL_PTRALIGN;
   if (!hs) return SMOE_EINVAL_NULL;
   if ((uintptr_t)hs & 3u) return SMOE_EINVAL_PTRALIGN;
-  if (small_gemm_rows(SmallWeights::kPacked, E, R))
+  if (small_gemm_rows(SmallWeights::kPacked, false, true, E, R, 2 * I, Kdim))
     return small_gemm_launch(SmallWeights::kPacked, false, a, as, w1p, w1s, offsets, E, R, 2 * I,
                              Kdim, c1, hq, hs, (hipStream_t)stream);
   long long mt_bound;

@@ -9,8 +9,9 @@ namespace smoe {
 
 enum class SmallWeights { kPacked, kPlain };
 
-// Whether a grouped GEMM of R rows over E experts takes the small-row kernel.
-bool small_gemm_rows(SmallWeights lay, int E, int R);
+// Whether a grouped GEMM of R rows over E experts, [N, K = Kdim] weights, takes
+// the small-row kernel (N = 2I in the fused SwiGLU form).
+bool small_gemm_rows(SmallWeights lay, bool e8m0, bool swiglu, int E, int R, int N, int Kdim);
 
 // The GEMM (hq == nullptr: c [R, N]) or, with hq, the fc1 GEMM with SwiGLU +
 // 1x128 requantisation (N = 2I; c1 into c when c is not null).  e8m0: every

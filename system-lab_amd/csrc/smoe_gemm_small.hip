@@ -10,16 +10,17 @@
 // expert every weight byte is used by one tile or two, and the time is that
 // of streaming the weights of the experts that have rows from HBM.
 //
-// Tiling.  A workgroup of 4 waves owns up to 96 rows x 64*kCB columns; wave w
+// Tiling.  A workgroup of 4 waves owns up to 112 rows (128 with E8M0 scales,
+// which need no registers for the MFMA's products) x 64*kCB columns; wave w
 // owns all rows and columns w*16*kCB .. +16*kCB.  The weights go straight
 // from memory to the MFMA operand registers (nothing else in the workgroup
 // needs them), kD K steps ahead.  The row count of a tile picks its loop: 1,
-// 2, 4 or 6 blocks of 16 rows, so a tile of one row does a sixteenth of a
-// 256-row tile's MFMAs.  The activations of a tile pass through LDS in chunks
+// 2, 4, 6 or 7 (8) blocks of 16 rows, so a tile of one row does a sixteenth of
+// a 256-row tile's MFMAs.  The activations of a tile pass through LDS in chunks
 // of at most 16 KiB (8, 4, 2 or 1 K steps), loaded to registers a chunk ahead
 // and written to the other half of the buffer at the chunk's end: one barrier
 // a chunk.  All loads are ordinary ones, so the compiler counts and waits for
-// each.  At most 256 registers and 51 KiB of LDS leave two workgroups per
+// each.  At most 256 registers and 68 KiB of LDS leave two workgroups per
 // CU, so one tile's start and end hide behind the other's stream.
 //
 // Every wave finds the workgroup's tile by itself (wave scans over the
@@ -34,13 +35,20 @@
 // of weights), fc2 162 -> 81 (5.8 TB/s); H 2048, I 768, E 128, top-8: fc1 with
 // SwiGLU 29 -> 20 at 1 token, 122 -> 70 at 64 (5.8 TB/s), 125 -> 97 at 1000;
 // its fc2 on plain weights 65 -> 40 at 64 tokens, with E8M0 scales 72 -> 33.
+// Tiles of up to 96 rows instead of 112 / 128: H = I = 2880, E 32, 777 tokens top-4
+// (97 rows) E8M0 fc1 151 -> 135, fc2 80 -> 62.  Loading the 64-row loop's weights
+// three steps ahead instead of two changed nothing but a 37-row case (5% slower).
 #include "smoe_gemm_small.h"
 #include "smoe_mfma.h"
 
 namespace smoe {
 namespace small {
 
-constexpr int kThreads = 256, kWaves = 4, kBM = 96;
+constexpr int kThreads = 256, kWaves = 4;
+// Most rows of a tile: what the registers hold beside two K steps of weights
+// (128 accumulators a lane, or 112 and the products the scales multiply).
+template <bool kE8>
+constexpr int kTileRows = kE8 ? 128 : 112;
 constexpr int kMaxChunk = 16 * 1024;  // most activation bytes of a chunk
 
 struct Tile {
@@ -49,10 +57,12 @@ struct Tile {
 
 // The tile of workgroup bid: false when it is past the last one.  offsets[] is
 // device data the host never sees: whatever it holds, rows stay in [0, R).
+template <int kBM>
 __device__ __forceinline__ bool find_tile(const int32_t* __restrict__ offsets, int E, int R, int NT,
                                           int mt_bound, int bid, int lane, Tile& t) {
+  auto row_at = [&](int e) { return max(0, min(offsets[min(e, E)], R)); };
   auto tiles = [&](int e) {
-    const int o0 = offsets[min(e, E)], o1 = offsets[min(e + 1, E)];
+    const int o0 = row_at(e), o1 = row_at(e + 1);
     return o1 > o0 ? min((o1 - o0 + kBM - 1) / kBM, mt_bound) : 0;
   };
   auto scan = [&](int v) {
@@ -112,11 +122,11 @@ __device__ __forceinline__ bool find_tile(const int32_t* __restrict__ offsets, i
   t.nt = q / nt_e;
   // the expert's n rows in nt_e = ceil(n / kBM) tiles of equal height, a
   // multiple of 16: at most kBM, so the last one is never empty
-  const int o0 = offsets[t.e], o1 = offsets[t.e + 1];
+  const int o0 = row_at(t.e), o1 = row_at(t.e + 1);
   const int h = min(((o1 - o0 + nt_e - 1) / nt_e + 15) & ~15, kBM);
   t.row0 = o0 + (q - t.nt * nt_e) * h;
-  t.rows = min(h, min(o1, R) - t.row0);
-  return t.row0 >= 0 && t.rows > 0;
+  t.rows = min(h, o1 - t.row0);
+  return t.rows > 0;
 }
 
 __device__ __forceinline__ int e8m0_of(float s) { return (__float_as_uint(s) >> 23) & 0xff; }
@@ -136,9 +146,10 @@ __device__ __forceinline__ void run_tile(const uint8_t* __restrict__ a_base,
                                          const float* __restrict__ sb_row, const uint32_t (&ob)[kCB],
                                          int rows, int Kd, int ksb, uint8_t* smem, int tid) {
   constexpr int kS = kRB <= 2 ? 8 / kRB : kRB == 4 ? 2 : 1;  // K steps per chunk
-  constexpr int kStep = kRB * 16 * kRow;  // LDS bytes per step
+  constexpr int kLB = kRB == 7 ? 8 : kRB;  // row blocks loaded: whole segments for every wave
+  constexpr int kStep = kLB * 16 * kRow;  // LDS bytes per step
   constexpr int kChunk = kS * kStep, kQ = kChunk / (kThreads * 16);
-  constexpr int kWords = kS * kRB * 16;  // activation scales of a chunk
+  constexpr int kWords = kS * kLB * 16;  // activation scales of a chunk
   constexpr bool kPacked = kLay == SmallWeights::kPacked;
   constexpr int kHalf = kPacked ? 1024 : 16;     // a weight fragment's second 16 bytes
   constexpr int kKStep = kPacked ? 2048 : kBK;   // weight bytes from one K block to the next
@@ -154,13 +165,13 @@ __device__ __forceinline__ void run_tile(const uint8_t* __restrict__ a_base,
 #pragma unroll
   for (int q = 0; q < kQ; ++q) {
     const int seg = q * kWaves + wid;
-    const int st = seg / (kRB * 2), rg = seg % (kRB * 2);
+    const int st = seg / (kLB * 2), rg = seg % (kLB * 2);
     const int row = tile_row(rg * 8 + (lane >> 3));
     oa[q] = (uint32_t)(min(row, rows - 1) * Kd + (((lane & 7) ^ (row & 7)) << 4));
     sa[q] = st;
   }
   // threads below kWords also carry one activation scale
-  const int s_row = tid % (kRB * 16), s_st = (tid / (kRB * 16)) % kS;
+  const int s_row = tid % (kLB * 16), s_st = (tid / (kLB * 16)) % kS;
   const uint32_t os = (uint32_t)(min(s_row, rows - 1) * ksb);
   v4i stg[kQ];
   float sstg;
@@ -210,7 +221,7 @@ __device__ __forceinline__ void run_tile(const uint8_t* __restrict__ a_base,
   auto step = [&](int kb, v8i (&f)[kCB]) {
     const int half = (kb / kS) & 1;
     const uint8_t* sA = smem + half * kChunk + (kb % kS) * kStep;
-    const float* sS = (const float*)(smem + 2 * kChunk) + half * kWords + (kb % kS) * kRB * 16;
+    const float* sS = (const float*)(smem + 2 * kChunk) + half * kWords + (kb % kS) * kLB * 16;
     const float sb = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(sbv), kb & 63));
     v8i fx = frag(sA, 0);
 #pragma unroll
@@ -284,7 +295,7 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_small_kernel(
     const float* __restrict__ bs, const int32_t* __restrict__ offsets, int E, int R, int N, int Kd,
     int mt_bound, uint16_t* __restrict__ c, uint8_t* __restrict__ hq, float* __restrict__ hs) {
   static_assert(!kSwiGLU || kCB == 4, "fused SwiGLU pairs 128 gate with 128 up columns");
-  constexpr int kBN = 64 * kCB, kCPitch = kBN * 2 + 16;
+  constexpr int kBN = 64 * kCB, kCPitch = kBN * 2 + 16, kBM = kTileRows<kE8>;
   constexpr int kLoop = 2 * kMaxChunk + 2 * kThreads * 4;
   constexpr int kSmem = kLoop > kBM * kCPitch ? kLoop : kBM * kCPitch;
   __shared__ __attribute__((aligned(1024))) uint8_t smem[kSmem];
@@ -293,7 +304,7 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_small_kernel(
   const int I = N / 2;
   const int NT = kSwiGLU ? I / kGroup : (N + kBN - 1) / kBN;
   Tile t;
-  if (!find_tile(offsets, E, R, NT, mt_bound, blockIdx.x, lane, t)) return;  // the whole workgroup leaves
+  if (!find_tile<kBM>(offsets, E, R, NT, mt_bound, blockIdx.x, lane, t)) return;  // the whole workgroup leaves
   const int e = t.e, row0 = t.row0, rows = t.rows, nt = t.nt;
   const int n0 = nt * kBN, ksb = Kd / kBK, NB = (N + kGroup - 1) / kGroup;
 
@@ -320,7 +331,8 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_small_kernel(
   if (rows <= 16) run_tile<kLay, kE8, kCB, 1, 4>(a_base, s_base, b_base, sb_row, ob, rows, Kd, ksb, smem, tid);
   else if (rows <= 32) run_tile<kLay, kE8, kCB, 2, 4>(a_base, s_base, b_base, sb_row, ob, rows, Kd, ksb, smem, tid);
   else if (rows <= 64) run_tile<kLay, kE8, kCB, 4, 2>(a_base, s_base, b_base, sb_row, ob, rows, Kd, ksb, smem, tid);
-  else run_tile<kLay, kE8, kCB, 6, 2>(a_base, s_base, b_base, sb_row, ob, rows, Kd, ksb, smem, tid);
+  else if (rows <= 96) run_tile<kLay, kE8, kCB, 6, 2>(a_base, s_base, b_base, sb_row, ob, rows, Kd, ksb, smem, tid);
+  else run_tile<kLay, kE8, kCB, kBM / 16, 2>(a_base, s_base, b_base, sb_row, ob, rows, Kd, ksb, smem, tid);
   __syncthreads();
 
   if constexpr (kSwiGLU) {
@@ -361,27 +373,61 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_small_kernel(
 
 }  // namespace small
 
-// The line between this kernel and the 256-row ones, on the average rows per
-// expert (the host knows no more).  Up to it an expert's rows mostly fit one
-// 96-row tile and its weights are streamed once; past it the second tile's
-// weights cost more than the 256-row tile's idle MFMAs.  Packed weights, fc1
-// with SwiGLU, 256-row kernel -> this one in us: 75 rows (H 4096, I 14336) 265
-// -> 182, 62 rows (H 2048, I 768) 125 -> 97, 65 rows (H 7168, I 2048) 241 ->
-// 182, but 100 rows of the last 253 -> 246 and their E8M0 form 223 -> 245.
-// Plain weights, whose fragment loads touch 16 lines each: 62 rows (H = I =
-// 2880) 165 -> 146, 97 rows 172 -> 188.  Under Zipf(1.2) loads the averages
-// below the line gain as much (65 rows: 246 -> 204 packed, 261 -> 245 plain),
-// and 88 rows lose (packed E8M0 227 -> 242, plain 269 -> 302).
-bool small_gemm_rows(SmallWeights lay, int E, int R) {
-  return R <= (lay == SmallWeights::kPacked ? 80LL : 64LL) * E;
+// The lines between this kernel and the 256-row ones, on the average rows per
+// expert (the host knows no more) and the shape.  256-row kernel -> this one in
+// us at random loads of the R rows.
+//
+// 1. One tile per expert: an expert's rows mostly fit one tile and its weights
+// are streamed once; past the line the second tile's pass over them costs more
+// than the 256-row tile's idle MFMAs.
+//   packed, 112 rows: N 1536, K 2048, E 128 150 -> 115; N 28672, K 4096, E 8 272 ->
+//     248; N 4096, K 7168, E 32 274 -> 257; at 192 rows 129 -> 148, 279 -> 274, 263 ->
+//     328
+//   packed E8M0, 112 rows: 122 -> 105, 251 -> 198, 230 -> 254 (at 100 rows 220 -> 191:
+//     512 tiles, two per CU); at 192 rows 126 -> 129, 261 -> 262, 239 -> 269
+//   N 4096, K 14336, E 8, few and long tiles: 75 rows 163 -> 131, 100 rows 163 -> 190
+//     (E8M0, whose tiles hold 128 rows: 158 -> 134)
+//   plain, whose fragment loads touch 16 lines each: 65 rows (N 4096, K 7168) 246 ->
+//     199, 97 rows (N 5760, K 2944) 153 -> 152, 100 rows (N 4096, K 7168) 249 -> 289
+// Zipf(1.2) loads below the line gain as much or more (packed 100 rows, N 4096,
+// K 7168: 301 -> 231; plain 75 rows 255 -> 256).
+//
+// 2. A chip that 256 x 256 tiles leave mostly idle, any rows per expert: up to 96
+// such tiles this kernel's more and smaller ones gain 1.04 - 2.7 (E 8, N 1024, 512
+// rows: K 2048 30.4 -> 25.6, K 4096 49.1 -> 41.2, plain 32.8 -> 29.1 and 55.5 -> 51.8),
+// at 112 0.83 - 1.11, from 144 on 0.63 - 1.07.  Not the plain SwiGLU form (0.91 - 1.36).
+//
+// 3. A short K in packed form, where a lone 256-row workgroup's prologue and
+// epilogue are most of its time and the second workgroup of a CU hides them
+// here.  Fused SwiGLU, whose epilogue is the longest:
+//   any rows: K <= 1536 1.05 - 1.43, E8M0 K <= 2048 1.02 - 1.9 (N 1536, E 128, 1024
+//     rows 1.14; N 768, 128 rows 0.95), both measured to 8192 rows
+//   256 - 1024 rows, a second and partly filled 256-row tile: K 2048 1.03 - 1.34
+//     (N 1536, E 128, 1024 rows 1.04), E8M0 K 2560 and 3072 1.01 - 1.36; above that
+//     0.96 - 1.03 and 0.93 - 1.07, at 192 rows (E8M0 K 2944) 0.92
+// and without the epilogue K < 1024: E8M0 to 1024 rows 1.01 - 1.48 (N 2048, K 768,
+// E 128: 512 rows 213 -> 195; at 2048 rows and N 256 0.86), K 512 to 512 rows 1.03 -
+// 1.53 (at 1024 rows 0.98).
+bool small_gemm_rows(SmallWeights lay, bool e8m0, bool swiglu, int E, int R, int N, int Kdim) {
+  const bool packed = lay == SmallWeights::kPacked;
+  const long long one_tile = !packed ? 80 : e8m0 || Kdim <= 8192 ? 112 : 80;
+  auto to = [&](long long rows) { return R <= rows * E; };
+  if (to(one_tile)) return true;
+  if ((packed || !swiglu) && (2LL * R + 256LL * E) * ((N + 255) / 256) <= 96 * 512) return true;
+  if (!packed) return false;
+  if (!swiglu) return Kdim < 1024 && to(e8m0 ? 1024 : 512);
+  if (Kdim <= (e8m0 ? 2048 : 1536)) return to(8192);
+  return Kdim <= (e8m0 ? 3072 : 2048) && R >= 256LL * E && to(1024);
 }
 
 int small_gemm_launch(SmallWeights lay, bool e8m0, const uint8_t* a, const float* as,
                       const uint8_t* b, const float* bs, const int32_t* offsets, int E, int R,
                       int N, int Kdim, uint16_t* c, uint8_t* hq, float* hs, hipStream_t stream) {
   // at most min(E, R) experts have rows, and each adds at most one partial tile
+  // to the R rows' whole ones (the slack serves offsets that overlap)
   const int live = E < R ? E : R;
-  const long long mt = live + (R - live) / small::kBM;
+  const int bm = e8m0 ? small::kTileRows<true> : small::kTileRows<false>;
+  const long long mt = live + ((long long)R + bm - 1) / bm;
   const bool swiglu = hq != nullptr;
   int cb = 4;
   if (!swiglu) {

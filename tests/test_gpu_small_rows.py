@@ -1,7 +1,7 @@
 """The grouped GEMM for few rows per expert (smoe_gemm_small.hip) against the
 256-row kernels, byte for byte: the same operands with unused rows past
-offsets[E], which push the average over the line, take the general path.
-The row counts sit on the edges of the 16-row blocks and of the 96-row tile,
+offsets[E], which push the average over every line, take the general path.
+The row counts sit on the edges of the 16-row blocks and of the 112 and 128-row tiles,
 K on both sides of the load-ahead and of the 64-step scale window, N on
 partial column tiles; more than 256 experts take the tile search's long
 form.  A CPU model checks the tile mapping for valid and malformed offsets."""
@@ -13,15 +13,14 @@ from oracle import smoe_oracle as O
 from smoe import ops
 from smoe import workloads as W
 
-BM = 96
 
 
 # ------------------------------------------------------------- CPU model
-def tiles(R, NT, offsets):
+def tiles(R, NT, offsets, BM):
     """(expert, first row, rows, column tile) of every workgroup that works."""
     E = len(offsets) - 1
-    live = min(E, R)
-    bound = live + (R - live) // BM
+    offsets = np.clip(offsets, 0, R)
+    bound = min(E, R) + -(-R // BM)
     cnt = [min(-(-max(0, int(offsets[e + 1]) - int(offsets[e])) // BM), bound) for e in range(E)]
     total = 0
     for b in range(0, E, 64):
@@ -41,8 +40,8 @@ def tiles(R, NT, offsets):
         o0, o1 = int(offsets[e]), int(offsets[e + 1])
         h = min((-(-(o1 - o0) // cnt[e]) + 15) & ~15, BM)
         row0 = o0 + (q - nt * cnt[e]) * h
-        rows = min(h, min(o1, R) - row0)
-        if row0 >= 0 and rows > 0:
+        rows = min(h, o1 - row0)
+        if rows > 0:
             out.append((e, row0, rows, nt))
     return out
 
@@ -58,7 +57,8 @@ def test_tiles_cover_every_row_once():
         off = lead + np.concatenate([[0], np.cumsum(counts)])
         NT = int(rng.integers(1, 4))
         seen = np.zeros((R, NT), int)
-        for e, row0, rows, nt in tiles(R, NT, off):
+        BM = int(rng.choice([112, 128]))
+        for e, row0, rows, nt in tiles(R, NT, off, BM):
             assert off[e] <= row0 and row0 + rows <= off[e + 1] and rows <= BM
             seen[row0:row0 + rows, nt] += 1
         assert (seen[off[0]:off[-1]] == 1).all() and seen.sum() == int(counts.sum()) * NT
@@ -69,8 +69,8 @@ def test_tiles_stay_in_range_for_malformed_offsets():
     for _ in range(200):
         E, R = int(rng.integers(1, 9)), int(rng.integers(1, 400))
         off = int(rng.integers(-300, 300)) + np.concatenate([[0], np.cumsum(rng.integers(-300, 900, E))])
-        for _, row0, rows, _ in tiles(R, 2, off):
-            assert 0 <= row0 and row0 + rows <= R and rows <= BM
+        for _, row0, rows, _ in tiles(R, 2, off, 112):
+            assert 0 <= row0 and row0 + rows <= R and rows <= 112
 
 
 # ------------------------------------------------------------------- GPU
@@ -82,7 +82,9 @@ def bits(t):
 CASES = [
     # counts, N, K: tile and block edges; K of 1, 3 and 5 steps, past 64 and 128 steps
     ([1, 15, 16, 17, 0, 31, 32, 33, 48, 49, 63, 64, 65], 512, 512),
-    ([95, 96, 97, 0, 2, 191, 0, 0, 192, 193, 1, 0, 0, 0, 0, 0], 256, 1024),
+    ([95, 96, 97, 0, 2, 111, 0, 0, 112, 113, 1, 0, 0, 0, 0, 0], 256, 1024),
+    ([127, 128, 129, 0, 224, 225, 256, 257, 3, 0, 0, 0, 0, 0], 256, 2048),
+    ([1500, 0, 700], 256, 1024),  # few tiles and a short K: many rows per expert
     ([5, 0, 20, 70], 272, 128),
     ([40, 3], 1040, 640),
     ([2, 0, 90, 33], 256, 66 * 128),
@@ -131,10 +133,11 @@ def test_small_rows_equal_the_256_row_kernels(dev, counts, N, K, form):
     xq, xs = ops.quant_rows(x, scale=scale)
     wq, ws = ops.quantize_weight_blockwise(W.weights(E, N, K, device=dev, seed=N), scale=scale)
     w = wq if form == "plain" else ops.pack_weight_fp8(wq)
-    big = 81 * E + n  # over the line: the 256-row kernels
     for swiglu in (False, True):
         if swiglu and N % 256:
             continue
+        # over the lines (1024 rows, 96 tiles; short K with SwiGLU 8192 rows): the 256-row kernels
+        big = n + max(1025 * E, 97 * 256) + (8192 * E if swiglu and K <= 2048 else 0)
         few = run(xq, xs, w, ws, off, n, e8m0, swiglu, N)
         for a, b in zip(few, run(xq, xs, w, ws, off, big, e8m0, swiglu, N)):
             assert torch.equal(a, b), f"swiglu={swiglu}"
