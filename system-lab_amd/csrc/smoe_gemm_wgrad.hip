@@ -51,66 +51,98 @@ enum WgradOut {
   kOutBF16Acc = SMOE_WGRAD_BF16_ACC
 };
 
-// One 256 x 256 tile of expert e's weight gradient at (n0, k0).  kE8M0: the
-// operands carry power-of-two scales (the optional E8M0 column recipe).
+// A 256 x 256 tile at (n0, k0) of expert e, whose row groups are steps groups
+// from column g0 of the operands.
+struct WTile {
+  int e, n0, k0, g0, steps;
+};
+
+// The stage of the coming tile's first row group, and whether it and the
+// tile's first scales are already there.
+struct WRing {
+  int buf;
+  bool ahead;
+};
+
+// One tile of the weight gradient.  kE8M0: the operands carry power-of-two
+// scales (the optional E8M0 column recipe).  The tile after it, next, has its
+// first row group and scales loaded during this tile's epilogue, whose stores
+// in turn drain during the next tile's first row group: a tile has only its
+// expert's rows / 128 steps, so its first load and its last store were up to a
+// third of its time.  us before -> now, E 128, N 1536, K 2048, 1024 rows per
+// expert: bf16 704 -> 653, added into 1064 -> 748 (the old values are read
+// while the pass is staged), fp32 777 -> 769, added into 1183 -> 950; E8M0 642 ->
+// 609, 995 -> 680, 711 -> 723, 1129 -> 911.  E 32, N = K = 2880, 512 rows: bf16
+// 341 -> 305, fp32 341 -> 341.  Loading the next tile during the last step
+// instead spilled (the loop body is at the register limit).
 template <int kOut, bool kE8M0>
 __device__ __forceinline__ void wgrad_tile(const uint8_t* __restrict__ aT,
                                            const float* __restrict__ aTs,
                                            const uint8_t* __restrict__ bT,
-                                           const float* __restrict__ bTs,
-                                           const int32_t* __restrict__ pad, int N, int Kd, int ld,
-                                           int e, int n0, int k0, uint8_t* smem,
-                                           void* __restrict__ dW) {
+                                           const float* __restrict__ bTs, int N, int Kd, int ld,
+                                           const WTile& cur, const WTile& next, WRing& ring,
+                                           uint8_t* smem, void* __restrict__ dW) {
   // opaque per tile: keeps lane-dependent address arithmetic inside the
   // caller's tile loop instead of live (in VGPRs) across it
   int tid = threadIdx.x;
   asm volatile("" : "+v"(tid));
   const int lane = tid & 63, wid = tid >> 6;
-  // operand columns outside [0, ld) are never read, whatever pad[] holds
-  const int g0 = max(pad[e], 0), g1 = min(pad[e + 1], ld);
-  const int steps = g1 > g0 ? (g1 - g0) / kGroup : 0;
+  const int e = cur.e, n0 = cur.n0, k0 = cur.k0, steps = cur.steps;
   const int nrows = min(kWN, N - n0), krows = min(kWK, Kd - k0);
   const int sld = ld / kGroup;  // scale row length
 
-  // DMA per wave and stage: aT segments w*4..w*4+3, bT segments w*4..w*4+3
-  // (8 rows of 128 bytes each).
-  // Lane offsets of segment j: row tile_row((wid*4+j)*8 + lane/8) clamped to
-  // the operand's rows, chunk (lane%8) ^ (row%8).  Recomputed at each issue
-  // (a few VALU operations) rather than held: the tile body needs the VGPRs.
-  auto seg_off = [&](int j, int lim) {
-    const int row = tile_row((wid * 4 + j) * 8 + (lane >> 3));
-    return (uint32_t)(min(row, lim - 1) * ld + (((lane & 7) ^ (row & 7)) << 4));
-  };
+  const int swid = __builtin_amdgcn_readfirstlane(wid);
   const uint32_t lds0 = (uint32_t)(uintptr_t)(lds_ptr_t)smem;
   // wave-uniform LDS destinations, computed once into scalar registers
   const uint32_t a_lds = __builtin_amdgcn_readfirstlane(lds0 + wid * 4 * 1024);
   const uint32_t b_lds = __builtin_amdgcn_readfirstlane(lds0 + kWA + wid * 4 * 1024);
-  auto issue = [&](int st_idx, int buf) {
-    const uint32_t st = buf * kWStage;
-    const int r0 = g0 + st_idx * kGroup;
-    const uint8_t* ab = aT + (size_t)n0 * ld + r0;
-    const uint8_t* bb = bT + (size_t)k0 * ld + r0;
+  // DMA per wave and stage: segments w*4..w*4+3 (8 row positions of 128 bytes
+  // each) of both operands.  Segment j's lane takes row tile_row((w*4 + j)*8 +
+  // lane/8) = w*32 + j/2*16 + j%2*4 + r0(lane), chunk (lane%8) ^ (row%8): two
+  // lane offsets serve a whole tile, the rest is in the scalar base.  A tile
+  // at the operand's edge clamps its rows, recomputed at each issue (opaque
+  // lane) rather than held: the K loop needs the VGPRs.
+  const int dr0 = (lane >> 4) + ((lane >> 3) & 1) * 8;
+  const uint32_t off0 = (uint32_t)(dr0 * ld + (((lane & 7) ^ (lane >> 4)) << 4));
+  auto issue_rows = [&](const uint8_t* b, int lim, uint32_t lds) {
+    if (lim == kWN) {
+      b += (size_t)(swid * 32) * ld;
 #pragma unroll
-    for (int j = 0; j < 4; ++j) dma16(ab, seg_off(j, nrows), a_lds + st + j * 1024);
+      for (int j = 0; j < 4; ++j)
+        dma16(b + (size_t)((j >> 1) * 16 + (j & 1) * 4) * ld, j & 1 ? off0 ^ 64u : off0, lds + j * 1024);
+    } else {
+      int ln = lane;
+      asm volatile("" : "+v"(ln));
 #pragma unroll
-    for (int j = 0; j < 4; ++j) dma16(bb, seg_off(j, krows), b_lds + st + j * 1024);
+      for (int j = 0; j < 4; ++j) {
+        const int row = tile_row((swid * 4 + j) * 8 + (ln >> 3));
+        dma16(b, (uint32_t)(min(row, lim - 1) * ld + (((ln & 7) ^ (row & 7)) << 4)), lds + j * 1024);
+      }
+    }
   };
-  // Scale chunk c (row groups g0/128 + 8c .. +8): waves 0-3 take aT rows
-  // (wid&3)*64 .., waves 4-7 bT rows; instruction i moves 8 rows x 8
-  // consecutive words (lane -> row i*8 + lane/8, group lane%8), so each
-  // instruction touches 8 short row segments instead of 64 rows.  Columns
-  // past the row end are clamped (their values are never used).
-  const float* sbase = uniform_ptr(wid < 4 ? aTs + (size_t)n0 * sld : bTs + (size_t)k0 * sld);
-  const int srows = wid < 4 ? nrows : krows;
+  auto issue = [&](const WTile& t, int st_idx, int buf) {
+    const uint32_t st = buf * kWStage;
+    const int r0 = t.g0 + st_idx * kGroup;
+    issue_rows(aT + (size_t)t.n0 * ld + r0, min(kWN, N - t.n0), a_lds + st);
+    issue_rows(bT + (size_t)t.k0 * ld + r0, min(kWK, Kd - t.k0), b_lds + st);
+  };
+  // Scale chunk c of a tile (row groups g0/128 + 8c .. +8) into LDS half h:
+  // waves 0-3 take aT rows (wid&3)*64 .., waves 4-7 bT rows; instruction i
+  // moves 8 rows x 8 consecutive words (lane -> row i*8 + lane/8, group
+  // lane%8), so each instruction touches 8 short row segments instead of 64
+  // rows.  Columns past the row end are clamped (their values are never used).
   const uint32_t sc_lds =
       __builtin_amdgcn_readfirstlane(lds0 + 2 * kWStage + wid * 64 * kWChunk * 4);
-  auto issue_sc = [&](int chunk) {
-    const int col = min(g0 / kGroup + chunk * kWChunk + (lane & 7), sld - 1);
+  auto issue_sc = [&](const WTile& t, int chunk, int h) {
+    const float* sbase = swid < 4 ? aTs + (size_t)t.n0 * sld : bTs + (size_t)t.k0 * sld;
+    const int srows = swid < 4 ? min(kWN, N - t.n0) : min(kWK, Kd - t.k0);
+    int ln = lane;
+    asm volatile("" : "+v"(ln));
+    const int col = min(t.g0 / kGroup + chunk * kWChunk + (ln & 7), sld - 1);
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
-      const int row = min((wid & 3) * 64 + i * 8 + (lane >> 3), srows - 1);
-      dma4(sbase, (uint32_t)(row * sld + col) * 4u,
-           sc_lds + (chunk & 1) * kWSC + i * 8 * kWChunk * 4);
+      const int row = min((swid & 3) * 64 + i * 8 + (ln >> 3), srows - 1);
+      dma4(sbase, (uint32_t)(row * sld + col) * 4u, sc_lds + h * kWSC + i * 8 * kWChunk * 4);
     }
   };
 
@@ -123,22 +155,22 @@ __device__ __forceinline__ void wgrad_tile(const uint8_t* __restrict__ aT,
 #pragma unroll
     for (int j = 0; j < 4; ++j) acc[i][j] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
 
-  if (steps > 0) {
-    issue_sc(0);
-    issue(0, 0);
+  if (steps > 0 && !ring.ahead) {
+    issue_sc(cur, 0, 0);
+    issue(cur, 0, ring.buf);
     __builtin_amdgcn_s_waitcnt(0);
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
   }
   for (int st = 0; st < steps; ++st) {
-    const int buf = st & 1;
+    const int buf = (ring.buf + st) & 1, half = (st / kWChunk) & 1;
     // the next scale chunk goes out at the first step of the current one,
     // into the half whose chunk was last read before the previous barrier
-    if ((st & (kWChunk - 1)) == 0 && st + kWChunk < steps) issue_sc(st / kWChunk + 1);
-    if (st + 1 < steps) issue(st + 1, buf ^ 1);
+    if ((st & (kWChunk - 1)) == 0 && st + kWChunk < steps) issue_sc(cur, st / kWChunk + 1, half ^ 1);
+    if (st + 1 < steps) issue(cur, st + 1, buf ^ 1);
     const uint8_t* sA = smem + buf * kWStage;
     const uint8_t* sB = sA + kWA;
-    const float* sSa = (const float*)(smem + 2 * kWStage + ((st / kWChunk) & 1) * kWSC) +
+    const float* sSa = (const float*)(smem + 2 * kWStage + half * kWSC) +
                        (st & (kWChunk - 1));
     const float* sSb = sSa + kWN * kWChunk;
     const int kr0 = wk * 128 + frow;
@@ -220,67 +252,119 @@ __device__ __forceinline__ void wgrad_tile(const uint8_t* __restrict__ aT,
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
   }
+  // the stage the last step read stages the output; the other one is the next tile's
+  uint8_t* out = smem + ((ring.buf + steps + 1) & 1) * kWStage;
+  ring.buf = (ring.buf + steps) & 1;
+  ring.ahead = next.steps > 0;
+  if (ring.ahead) {
+    issue_sc(next, 0, 0);
+    issue(next, 0, ring.buf);
+  }
 
   // An expert without rows adds nothing to an accumulation buffer.
-  if ((kOut == kOutF32Acc || kOut == kOutBF16Acc) && steps == 0) return;
+  if ((kOut == kOutF32Acc || kOut == kOutBF16Acc) && steps == 0) {
+    __builtin_amdgcn_s_waitcnt(0);
+    asm volatile("s_barrier" ::: "memory");
+    return;
+  }
 
-  // Epilogue: the fp32 tile leaves through LDS in two 128-row halves (the
-  // stage buffers are free after the K loop's last barrier).  Lane (i, j)
-  // holds dW row n = wn*64 + j*16 + lane%16, columns k = wk*128 + i*16 +
-  // (lane/16)*4 .. +3, written as one 16-byte word; with a row pitch of 260
-  // floats the 16 rows of a lane group start 4 banks apart, so each group's
-  // 16-byte writes cover all 64 banks once (conflict-free).  Then each
-  // wave writes whole rows, 4 columns per lane: fp32 as 16-byte stores,
-  // non-temporal (dW is written once here and read by a later kernel), bf16
-  // rounded to nearest even as 8-byte stores.  The accumulating modes read
-  // the 4 columns first and add the tile's fp32 values to them (one fp32
-  // addition per value, then the bf16 rounding for a bf16 buffer: the same
-  // result as adding an fp32 gradient to the buffer in a separate pass).
-  float* ct = (float*)smem;
-  constexpr int kPitch = kWK + 4;
-  static_assert(128 * kPitch * 4 <= kWSmem, "epilogue half-tile fits the LDS buffers");
+  // Epilogue: the tile leaves through one 64 KiB stage in passes of kPass rows,
+  // as many from every wave: 128 rows of bf16 (rounded to nearest even as they
+  // are staged), or 64 of fp32.  Lane (i, j) holds dW row n = wn*64 + j*16 +
+  // lane%16, columns k = wk*128 + i*16 + (lane/16)*4 .. +3; pass p takes j =
+  // p*kJ .. +kJ.  Staged row r holds its 16-byte chunk c at c ^ (r % 16), so
+  // the 16 rows of a block write every bank once.  Each wave then reads its 8
+  // KiB of the pass and writes whole rows, 16 bytes per lane: fp32 non-temporal (dW is written once here and read by a
+  // later kernel).  The accumulating modes read dW while the pass is staged
+  // and add the tile's fp32 values to it (one fp32 addition per value, then
+  // the bf16 rounding for a bf16 buffer: the same result as adding an fp32
+  // gradient to the buffer in a separate pass).
+  constexpr bool kHalf = kOut == kOutBF16;
+  constexpr bool kAcc = kOut == kOutF32Acc || kOut == kOutBF16Acc;
+  constexpr int kJ = kHalf ? 2 : 1, kPass = 64 * kJ;
+  constexpr int kRowBytes = kWK * (kHalf ? 2 : 4);
+  static_assert(kPass * kRowBytes == kWStage, "a pass fills a stage");
+  // Staged row r is output row row_of(p, r): kJ*16 rows of each wave quarter.
+  // A lane writes 16 bytes (8 or 4 columns) of kIt rows.
+  auto row_of = [&](int p, int r) { return r / (16 * kJ) * 64 + p * 16 * kJ + r % (16 * kJ); };
+  constexpr bool kOut16 = kOut == kOutBF16 || kOut == kOutBF16Acc;
+  constexpr int kIt = kPass * kWK * (kOut16 ? 2 : 4) / (kWThreads * 16);
+  const int lrow = kOut16 ? wid * 2 + (lane >> 5) : wid, lc = kOut16 ? lane & 31 : lane;
+  constexpr int kLRows = kOut16 ? 16 : 8, kCols = kOut16 ? 8 : 4;
 #pragma unroll
-  for (int half = 0; half < 2; ++half) {
-    if ((wn >> 1) == half) {
+  for (int p = 0; p < kWN / kPass; ++p) {
+    // the lane's piece of dW at row it: null past the edge
+    auto piece = [&](int it) -> v4i* {
+      const int nl = row_of(p, it * kLRows + lrow);
+      if (nl >= nrows || lc * kCols >= krows) return nullptr;
+      const size_t o = ((size_t)e * N + n0 + nl) * Kd + k0 + lc * kCols;
+      return (v4i*)((uint8_t*)dW + o * (kOut16 ? 2 : 4));
+    };
+    v4i old[kIt];
+    if constexpr (kAcc) {
 #pragma unroll
-      for (int i = 0; i < 8; ++i)
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          const int row = (wn & 1) * 64 + j * 16 + frow;
-          *(v4f*)(ct + row * kPitch + wk * 128 + i * 16 + (lane >> 4) * 4) = acc[i][j];
-        }
+      for (int it = 0; it < kIt; ++it)
+        if (const v4i* d = piece(it)) old[it] = *d;
     }
-    __syncthreads();
-    for (int r = wid; r < 128; r += 8) {
-      const int nl = half * 128 + r;
-      if (nl < nrows && lane * 4 < krows) {
-        v4f val = *(const v4f*)(ct + r * kPitch + lane * 4);
-        const size_t o = ((size_t)e * N + n0 + nl) * Kd + k0 + lane * 4;
-        if constexpr (kOut == kOutF32) {
-          __builtin_nontemporal_store(val, (v4f*)((float*)dW + o));
-        } else if constexpr (kOut == kOutF32Acc) {
-          v4f* d = (v4f*)((float*)dW + o);
-          const v4f old = *d;
 #pragma unroll
-          for (int v = 0; v < 4; ++v) val[v] = old[v] + val[v];
-          *d = val;
-        } else {
-          uint2* d = (uint2*)((uint16_t*)dW + o);
-          if constexpr (kOut == kOutBF16Acc) {
-            const uint2 old = *d;
-            val[0] += __uint_as_float(old.x << 16);
-            val[1] += __uint_as_float(old.x & 0xffff0000u);
-            val[2] += __uint_as_float(old.y << 16);
-            val[3] += __uint_as_float(old.y & 0xffff0000u);
-          }
+    for (int jj = 0; jj < kJ; ++jj)
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        const v4f v = acc[i][p * kJ + jj];
+        const int c = kHalf ? (wk * 8 + i) * 2 + (lane >> 5) : (wk * 8 + i) * 4 + (lane >> 4);
+        uint8_t* d = out + (wn * 16 * kJ + jj * 16 + frow) * kRowBytes + ((c ^ frow) << 4);
+        if constexpr (kHalf) {
           uint2 b;
-          b.x = bf16_pack2(val[0], val[1]);
-          b.y = bf16_pack2(val[2], val[3]);
-          *d = b;
+          b.x = bf16_pack2(v[0], v[1]);
+          b.y = bf16_pack2(v[2], v[3]);
+          *(uint2*)(d + ((lane >> 4) & 1) * 8) = b;
+        } else {
+          *(v4f*)d = v;
         }
       }
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    constexpr int kSt = kWStage / (kWThreads * 16);  // this wave's 8 KiB of the pass, read at once
+    v4f st[kSt];
+#pragma unroll
+    for (int it = 0; it < kSt; ++it) {
+      // (bf16 added into: two chunks of fp32 make a lane's 8 columns)
+      const int r = (kSt == kIt ? it : it / 2) * kLRows + lrow, c = kSt == kIt ? lc : lc * 2 + it % 2;
+      st[it] = *(const v4f*)(out + r * kRowBytes + ((c ^ (r & 15)) << 4));
     }
-    __syncthreads();
+#pragma unroll
+    for (int it = 0; it < kIt; ++it) {
+      v4i* d = piece(it);
+      if (!d) continue;
+      if constexpr (kOut == kOutF32) {
+        __builtin_nontemporal_store(st[it], (v4f*)d);
+      } else if constexpr (kOut == kOutBF16) {
+        *(v4f*)d = st[it];
+      } else if constexpr (kOut == kOutF32Acc) {
+        v4f b;
+#pragma unroll
+        for (int v = 0; v < 4; ++v) b[v] = __int_as_float(old[it][v]) + st[it][v];
+        *(v4f*)d = b;
+      } else {
+        v4i b;
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+          const uint32_t w = (uint32_t)old[it][v];
+          const v4f s = st[it * 2 + v / 2];
+          b[v] = (int)bf16_pack2(__uint_as_float(w << 16) + s[v % 2 * 2],
+                                 __uint_as_float(w & 0xffff0000u) + s[v % 2 * 2 + 1]);
+        }
+        *d = b;
+      }
+    }
+    if (p + 1 == kWN / kPass && ring.ahead) {
+      // the next tile's loads are in LDS: they are older than the stores, of
+      // which a wave of a whole tile issued kIt a pass
+      static_assert(kIt * (kWN / kPass) == (kOut16 ? 16 : 32), "stores of a wave");
+      if (nrows < kWN || krows < kWK) __builtin_amdgcn_s_waitcnt(0);
+      else if constexpr (kOut16) asm volatile("s_waitcnt vmcnt(16)" ::: "memory");
+      else asm volatile("s_waitcnt vmcnt(32)" ::: "memory");
+    }
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
   }
 }
 
@@ -365,12 +449,26 @@ __global__ __launch_bounds__(kWThreads, 1) void grouped_gemm_fp8_wgrad_kernel(
   const int t_end =
       __builtin_amdgcn_readfirstlane(xcd == 7 ? E * TE : (int)first_tile(W * (xcd + 1) / 8));
   __syncthreads();  // the tiles' DMA overwrites the cost table
+  auto tile_of = [&](int t) {
+    WTile w{};
+    if (t < t_end) {
+      w.e = t / TE;
+      const int rem = t - w.e * TE;
+      w.n0 = rem / KT * kWN;
+      w.k0 = rem % KT * kWK;
+      // operand columns outside [0, ld) are never read, whatever pad[] holds
+      w.g0 = max(pad[w.e], 0);
+      const int g1 = min(pad[w.e + 1], ld);
+      w.steps = g1 > w.g0 ? (g1 - w.g0) / kGroup : 0;
+    }
+    return w;
+  };
+  WRing ring{0, false};
+  WTile cur = tile_of(t_begin + j);
   for (int t = t_begin + j; t < t_end; t += per_xcd) {
-    const int e = t / TE;
-    const int rem = t - e * TE;
-    wgrad_tile<kOut, kE8M0>(aT, aTs, bT, bTs, pad, N, Kd, ld, e, (rem / KT) * kWN, (rem % KT) * kWK, smem,
-                     dW);
-    __syncthreads();  // the next tile reuses the LDS
+    const WTile next = tile_of(t + per_xcd);
+    wgrad_tile<kOut, kE8M0>(aT, aTs, bT, bTs, N, Kd, ld, cur, next, ring, smem, dW);
+    cur = next;
   }
 }
 
