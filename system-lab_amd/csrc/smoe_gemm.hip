@@ -41,6 +41,8 @@
 #include "smoe_gemm_small.h"
 #include "smoe_mfma.h"
 
+#include <type_traits>
+
 namespace smoe {
 
 // m-tiles per chip-wide scheduling group: 4 per XCD, so an XCD's 32 CUs run
@@ -78,7 +80,7 @@ struct Cfg {
 // when not null.  h is computed from the bf16-rounded fc1 values exactly as
 // the stand-alone SwiGLU kernel does, so the fused path is bit-identical to
 // GEMM -> bf16 c1 -> swiglu_quant.
-template <class C, bool kSwiGLU, bool kChunkS>
+template <class C, bool kSwiGLU, bool kChunkS, bool kShort>
 __global__ __launch_bounds__(C::kThreads, 1) void grouped_gemm_fp8_kernel(
     const uint8_t* __restrict__ a, const float* __restrict__ as, const uint8_t* __restrict__ b,
     const float* __restrict__ bs, const int32_t* __restrict__ offsets, int E, int R, int N,
@@ -284,6 +286,13 @@ __global__ __launch_bounds__(C::kThreads, 1) void grouped_gemm_fp8_kernel(
   __builtin_amdgcn_s_barrier();
   asm volatile("" ::: "memory");
 
+  // kShort: an expert's last tile has fewer rows; waves whose 128 rows are
+  // empty skip the step's MFMAs, waves with at most 64 half of them.  us without
+  // -> with: E 32, N 5760, K 2944 157 -> 130 (97 rows per expert), 292 -> 266 (312);
+  // N 4096, K 7168 264 -> 247 (150), 578 -> 561 (500); E 128, N 2048, K 768 81 -> 75
+  // (128), 196 -> 188 (512); N 2048, K 7168, 8192 rows under Zipf(1.2) 221 -> 201;
+  // from 2048 rows on nothing.
+  const int wrows = kShort ? __builtin_amdgcn_readfirstlane(rows - wr * kRB * 16) : kRB * 16;
   int buf = 0;
   for (int kb = 0; kb < ksb; ++kb) {
     // refill the slot consumed in the previous step (free after its barrier)
@@ -297,26 +306,31 @@ __global__ __launch_bounds__(C::kThreads, 1) void grouped_gemm_fp8_kernel(
     const float* sS = (const float*)(sB + kBBytes);
     const float* sC = (const float*)(smem + kSC0 + ((kb / kSChunk) & 1) * kSCBytes) + (kb & (kSChunk - 1));
     const float sb = sb_row[kb];
-    v8i fw[4];
+    auto compute = [&](auto m) __attribute__((always_inline)) {
+      constexpr int kM = decltype(m)::value;  // the wave's row blocks with rows
+      v8i fw[4];
 #pragma unroll
-    for (int j = 0; j < 4; ++j) fw[j] = lds_frag(sB, wn * 64 + j * 16 + frow, fch);
-    // the next row block's activation fragment is read before this block's
-    // MFMAs are issued, so its LDS latency hides behind them
-    const int rbase = wr * kRB * 16 + frow;
-    v8i fx = lds_frag(sA, rbase, fch);
+      for (int j = 0; j < 4; ++j) fw[j] = lds_frag(sB, wn * 64 + j * 16 + frow, fch);
+      // the next row block's activation fragment is read before this block's
+      // MFMAs are issued, so its LDS latency hides behind them
+      const int rbase = wr * kRB * 16 + frow;
+      v8i fx = lds_frag(sA, rbase, fch);
 #pragma unroll
-    for (int i = 0; i < kRB; ++i) {
-      v8i fxn = fx;
-      if (i + 1 < kRB) fxn = lds_frag(sA, rbase + (i + 1) * 16, fch);
-      const float sc = (kChunkS ? sC[(rbase + i * 16) * kSChunk] : sS[rbase + i * 16]) * sb;
+      for (int i = 0; i < kM; ++i) {
+        v8i fxn = fx;
+        if (i + 1 < kM) fxn = lds_frag(sA, rbase + (i + 1) * 16, fch);
+        const float sc = (kChunkS ? sC[(rbase + i * 16) * kSChunk] : sS[rbase + i * 16]) * sb;
 #pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const v4f p = mfma16(fw[j], fx, v4f{0.0f, 0.0f, 0.0f, 0.0f});
+        for (int j = 0; j < 4; ++j) {
+          const v4f p = mfma16(fw[j], fx, v4f{0.0f, 0.0f, 0.0f, 0.0f});
 #pragma unroll
-        for (int v = 0; v < 4; ++v) acc[i][j][v] = __builtin_fmaf(p[v], sc, acc[i][j][v]);
+          for (int v = 0; v < 4; ++v) acc[i][j][v] = __builtin_fmaf(p[v], sc, acc[i][j][v]);
+        }
+        fx = fxn;
       }
-      fx = fxn;
-    }
+    };
+    if (!kShort || wrows > kRB * 8) compute(std::integral_constant<int, kRB>{});
+    else if (wrows > 0) compute(std::integral_constant<int, kRB / 2>{});
     // stage kb+1 must have landed for every wave; later stages may still fly
     if (kStages > 2 && kb + kStages - 1 < ksb) {
       if (scale_wave) wait_vm_lgkm0<kASegs + kBSegs + 1>();
@@ -382,6 +396,24 @@ __global__ __launch_bounds__(C::kThreads, 1) void grouped_gemm_fp8_kernel(
 #endif
 using GemmCfg = SMOE_GEMM_CFG;
 
+// The instantiation of one call: the scale staging by K, the short tiles by
+// load.  The SwiGLU form with staged scales has no registers left for them (5
+// spills: N 4096, K 7168, 500 rows per expert 612 -> 680 us).
+#define SMOE_PLAIN_K(SW, CH, SH, W, WS, ...)                                                 \
+  grouped_gemm_fp8_kernel<C, SW, CH, SH>                                                     \
+      <<<dim3((unsigned)nblk), dim3(C::kThreads), 0, (hipStream_t)stream>>>(                 \
+          a, as, W, WS, offsets, E, R, N, Kdim, (int)mt_bound, __VA_ARGS__)
+#define SMOE_PLAIN(SW, W, WS, ...)                                      \
+  do {                                                                  \
+    const bool chunk = Kdim % (kBK * 4) == 0;                           \
+    const bool cut = !(SW && chunk) && short_tiles(E, R, NT, 256, 256, 1024); \
+    if (cut && chunk) SMOE_PLAIN_K(SW, true, !SW, W, WS, __VA_ARGS__);  \
+    else if (cut) SMOE_PLAIN_K(SW, false, true, W, WS, __VA_ARGS__);    \
+    else if (chunk) SMOE_PLAIN_K(SW, true, false, W, WS, __VA_ARGS__);  \
+    else SMOE_PLAIN_K(SW, false, false, W, WS, __VA_ARGS__);            \
+    SMOE_RETURN_LAUNCH();                                               \
+  } while (0)
+
 }  // namespace smoe
 
 using namespace smoe;
@@ -417,15 +449,7 @@ extern "C" int smoe_grouped_gemm_fp8(const uint8_t* a, const float* as, const ui
   long long nblk = mt_pad * NT;
   nblk = (nblk + 7) / 8 * 8;
   if (nblk > 0x7fffffffLL) return SMOE_EINVAL_DIM;
-  if (Kdim % (kBK * 4) == 0)
-    grouped_gemm_fp8_kernel<C, false, true>
-        <<<dim3((unsigned)nblk), dim3(C::kThreads), 0, (hipStream_t)stream>>>(
-            a, as, b, bs, offsets, E, R, N, Kdim, (int)mt_bound, c, nullptr, nullptr);
-  else
-    grouped_gemm_fp8_kernel<C, false, false>
-        <<<dim3((unsigned)nblk), dim3(C::kThreads), 0, (hipStream_t)stream>>>(
-            a, as, b, bs, offsets, E, R, N, Kdim, (int)mt_bound, c, nullptr, nullptr);
-  SMOE_RETURN_LAUNCH();
+  SMOE_PLAIN(false, b, bs, c, nullptr, nullptr);
 }
 
 extern "C" int smoe_grouped_gemm_fp8_swiglu(const uint8_t* a, const float* as, const uint8_t* w1,
@@ -456,13 +480,5 @@ extern "C" int smoe_grouped_gemm_fp8_swiglu(const uint8_t* a, const float* as, c
   long long nblk = mt_pad * NT;
   nblk = (nblk + 7) / 8 * 8;
   if (nblk > 0x7fffffffLL) return SMOE_EINVAL_DIM;
-  if (Kdim % (kBK * 4) == 0)
-    grouped_gemm_fp8_kernel<C, true, true>
-        <<<dim3((unsigned)nblk), dim3(C::kThreads), 0, (hipStream_t)stream>>>(
-            a, as, w1, w1s, offsets, E, R, N, Kdim, (int)mt_bound, c1, hq, hs);
-  else
-    grouped_gemm_fp8_kernel<C, true, false>
-        <<<dim3((unsigned)nblk), dim3(C::kThreads), 0, (hipStream_t)stream>>>(
-            a, as, w1, w1s, offsets, E, R, N, Kdim, (int)mt_bound, c1, hq, hs);
-  SMOE_RETURN_LAUNCH();
+  SMOE_PLAIN(true, w1, w1s, c1, hq, hs);
 }

@@ -32,6 +32,8 @@
 #include "smoe_gemm_small.h"
 #include "smoe_mfma.h"
 
+#include <type_traits>
+
 namespace smoe {
 namespace e8m0 {
 
@@ -96,7 +98,7 @@ __device__ __forceinline__ void mfma_scale_acc(v4f& acc, const v8i& a, const v8i
 // and the epilogue writes h = silu(gate) * up requantised 1x128 with
 // power-of-two scales into hq [R, I], hs [R, I/128] (and c1 when c is not
 // null): the bytes of the SwiGLU quantiser run on this kernel's c.
-template <bool kSwiGLU>
+template <bool kSwiGLU, bool kShort>
 __global__ __launch_bounds__(kThreads, 1) void grouped_gemm_fp8_e8m0_kernel(
     const uint8_t* __restrict__ a, const float* __restrict__ as, const uint8_t* __restrict__ bp,
     const float* __restrict__ bs, const int32_t* __restrict__ offsets, int E, int R, int N, int Kd,
@@ -301,7 +303,8 @@ __global__ __launch_bounds__(kThreads, 1) void grouped_gemm_fp8_e8m0_kernel(
   // and the weights of step kb+1, both needed within the next step) and
   // leaves step kb-1's loads in flight.  Past the last step the loads repeat
   // step ksb-1's data into buffers and stages no later step reads.
-  auto step = [&](int kb, WBuf& cur, WBuf& nxt, bool tail) __attribute__((always_inline)) {
+  auto step = [&](auto m, int kb, WBuf& cur, WBuf& nxt, bool tail) __attribute__((always_inline)) {
+    constexpr int kM = decltype(m)::value;  // row blocks with rows: 16, 8 or 4
     const int ka = min(kb + kAS - 1, ksb - 1);
     const uint32_t a_dst = a_lds + (uint32_t)((kb + kAS - 1) % kAS) * kABytes;
     const uint8_t* a_src = a_base + (size_t)ka * kBK;
@@ -320,16 +323,20 @@ __global__ __launch_bounds__(kThreads, 1) void grouped_gemm_fp8_e8m0_kernel(
     v8i fx = lds_frag_p(sA, frow, fg);
     int ex = e8m0_of(sC[frow * kSChunk]);
 #pragma unroll
-    for (int i = 0; i < kRB; ++i) {
-      if (i < 8) {
-        dma16(a_src, oa[i], a_dst + i * 1024);
-      } else {
-        const int q = i - 8;  // weight load q: column block q >> 1, half q & 1
-        nxt[q >> 1][q & 1] = *(const v4i*)(b_src + ob[q >> 1] + (q & 1) * 1024);
+    for (int i = 0; i < kM; ++i) {
+      // the step's 16 loads, 16 / kM before each row block
+#pragma unroll
+      for (int l = i * (16 / kM); l < (i + 1) * (16 / kM); ++l) {
+        if (l < 8) {
+          dma16(a_src, oa[l], a_dst + l * 1024);
+        } else {
+          const int q = l - 8;  // weight load q: column block q >> 1, half q & 1
+          nxt[q >> 1][q & 1] = *(const v4i*)(b_src + ob[q >> 1] + (q & 1) * 1024);
+        }
       }
       v8i fxn = fx;
       int exn = ex;
-      if (i + 1 < kRB) {
+      if (i + 1 < kM) {
         fxn = lds_frag_p(sA, (i + 1) * 16 + frow, fg);
         exn = e8m0_of(sC[((i + 1) * 16 + frow) * kSChunk]);
       }
@@ -352,16 +359,26 @@ __global__ __launch_bounds__(kThreads, 1) void grouped_gemm_fp8_e8m0_kernel(
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
   };
-  int kb = 0;
-  for (; kb + 3 < ksb; kb += 4) {
-    step(kb, fA, fD, false);
-    step(kb + 1, fB, fA, false);
-    step(kb + 2, fC, fB, false);
-    step(kb + 3, fD, fC, false);
-  }
-  if (kb < ksb) step(kb, fA, fD, true);
-  if (kb + 1 < ksb) step(kb + 1, fB, fA, true);
-  if (kb + 2 < ksb) step(kb + 2, fC, fB, true);
+  auto k_loop = [&](auto m) __attribute__((always_inline)) {
+    int kb = 0;
+    for (; kb + 3 < ksb; kb += 4) {
+      step(m, kb, fA, fD, false);
+      step(m, kb + 1, fB, fA, false);
+      step(m, kb + 2, fC, fB, false);
+      step(m, kb + 3, fD, fC, false);
+    }
+    if (kb < ksb) step(m, kb, fA, fD, true);
+    if (kb + 1 < ksb) step(m, kb + 1, fB, fA, true);
+    if (kb + 2 < ksb) step(m, kb + 2, fC, fB, true);
+  };
+  // kShort: an expert's last tile has fewer rows, and its empty row blocks are
+  // skipped.  us without -> with: E 32, N 5760, K 2944 263 -> 244 (312 rows per
+  // expert), 354 -> 334 (512); N 4096, K 7168 303 -> 297 (250), 1660 -> 1612 (2048); E
+  // 128, N 1536, K 2048 173 -> 168 (256), 471 -> 461 (1024); between 128 and 256 rows,
+  // where few tiles are short, up to 3% slower.
+  if (!kShort || rows > 128) k_loop(std::integral_constant<int, kRB>{});
+  else if (rows > 64) k_loop(std::integral_constant<int, 8>{});
+  else k_loop(std::integral_constant<int, 4>{});
   asm volatile("s_nop 15\n\ts_nop 15" ::: "memory");  // last MFMA results settle
   wait_vm<0>();
   __syncthreads();
@@ -450,9 +467,14 @@ extern "C" int smoe_grouped_gemm_fp8_packed_e8m0(const uint8_t* a, const float* 
   long long mt_bound;
   const long long nblk = e8m0_grid(E, R, (N + e8m0::kBN - 1) / e8m0::kBN, &mt_bound);
   if (nblk > 0x7fffffffLL) return SMOE_EINVAL_DIM;
-  e8m0::grouped_gemm_fp8_e8m0_kernel<false>
-      <<<dim3((unsigned)nblk), dim3(e8m0::kThreads), 0, (hipStream_t)stream>>>(
-          a, as, wp, ws, offsets, E, R, N, Kdim, (int)mt_bound, c, nullptr, nullptr);
+  if (short_tiles(E, R, (N + e8m0::kBN - 1) / e8m0::kBN, 128, 256, 2048))
+    e8m0::grouped_gemm_fp8_e8m0_kernel<false, true>
+        <<<dim3((unsigned)nblk), dim3(e8m0::kThreads), 0, (hipStream_t)stream>>>(
+            a, as, wp, ws, offsets, E, R, N, Kdim, (int)mt_bound, c, nullptr, nullptr);
+  else
+    e8m0::grouped_gemm_fp8_e8m0_kernel<false, false>
+        <<<dim3((unsigned)nblk), dim3(e8m0::kThreads), 0, (hipStream_t)stream>>>(
+            a, as, wp, ws, offsets, E, R, N, Kdim, (int)mt_bound, c, nullptr, nullptr);
   SMOE_RETURN_LAUNCH();
 }
 
@@ -475,8 +497,13 @@ extern "C" int smoe_grouped_gemm_fp8_packed_e8m0_swiglu(const uint8_t* a, const 
   long long mt_bound;
   const long long nblk = e8m0_grid(E, R, I / kGroup, &mt_bound);
   if (nblk > 0x7fffffffLL) return SMOE_EINVAL_DIM;
-  e8m0::grouped_gemm_fp8_e8m0_kernel<true>
-      <<<dim3((unsigned)nblk), dim3(e8m0::kThreads), 0, (hipStream_t)stream>>>(
-          a, as, w1p, w1s, offsets, E, R, 2 * I, Kdim, (int)mt_bound, c1, hq, hs);
+  if (short_tiles(E, R, I / kGroup, 128, 256, 2048))
+    e8m0::grouped_gemm_fp8_e8m0_kernel<true, true>
+        <<<dim3((unsigned)nblk), dim3(e8m0::kThreads), 0, (hipStream_t)stream>>>(
+            a, as, w1p, w1s, offsets, E, R, 2 * I, Kdim, (int)mt_bound, c1, hq, hs);
+  else
+    e8m0::grouped_gemm_fp8_e8m0_kernel<true, false>
+        <<<dim3((unsigned)nblk), dim3(e8m0::kThreads), 0, (hipStream_t)stream>>>(
+            a, as, w1p, w1s, offsets, E, R, 2 * I, Kdim, (int)mt_bound, c1, hq, hs);
   SMOE_RETURN_LAUNCH();
 }

@@ -383,14 +383,15 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_small_kernel(
 //   packed, 112 rows: N 1536, K 2048, E 128 150 -> 115; N 28672, K 4096, E 8 272 ->
 //     248; N 4096, K 7168, E 32 274 -> 257; at 192 rows 129 -> 148, 279 -> 274, 263 ->
 //     328
-//   packed E8M0, 112 rows: 122 -> 105, 251 -> 198, 230 -> 254 (at 100 rows 220 -> 191:
-//     512 tiles, two per CU); at 192 rows 126 -> 129, 261 -> 262, 239 -> 269
-//   N 4096, K 14336, E 8, few and long tiles: 75 rows 163 -> 131, 100 rows 163 -> 190
-//     (E8M0, whose tiles hold 128 rows: 158 -> 134)
+//   packed E8M0, whose 256-row kernel skips empty row blocks, 112 rows: 111 -> 105,
+//     212 -> 198, 204 -> 254 (at 88 rows and Zipf loads 218 -> 235); at 192 rows 126 ->
+//     129, 261 -> 262, 239 -> 269
+//   N 4096, K 14336, E 8, few and long tiles: 75 rows 163 -> 131, 100 rows 163 -> 190,
+//     E8M0 112 rows 132 -> 141, 75 rows and Zipf loads 158 -> 181
 //   plain, whose fragment loads touch 16 lines each: 65 rows (N 4096, K 7168) 246 ->
-//     199, 97 rows (N 5760, K 2944) 153 -> 152, 100 rows (N 4096, K 7168) 249 -> 289
+//     199, 97 rows (N 5760, K 2944) 130 -> 152, 100 rows (N 4096, K 7168) 249 -> 289
 // Zipf(1.2) loads below the line gain as much or more (packed 100 rows, N 4096,
-// K 7168: 301 -> 231; plain 75 rows 255 -> 256).
+// K 7168: 291 -> 227; plain 75 rows 259 -> 259).
 //
 // 2. A chip that 256 x 256 tiles leave mostly idle, any rows per expert: up to 96
 // such tiles this kernel's more and smaller ones gain 1.04 - 2.7 (E 8, N 1024, 512
@@ -410,7 +411,9 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_small_kernel(
 // 1.53 (at 1024 rows 0.98).
 bool small_gemm_rows(SmallWeights lay, bool e8m0, bool swiglu, int E, int R, int N, int Kdim) {
   const bool packed = lay == SmallWeights::kPacked;
-  const long long one_tile = !packed ? 80 : e8m0 || Kdim <= 8192 ? 112 : 80;
+  const long long one_tile = !packed ? 80
+                             : e8m0  ? (Kdim <= 4096 ? 112 : Kdim <= 8192 ? 80 : 64)
+                                     : (Kdim <= 8192 ? 112 : 80);
   auto to = [&](long long rows) { return R <= rows * E; };
   if (to(one_tile)) return true;
   if ((packed || !swiglu) && (2LL * R + 256LL * E) * ((N + 255) / 256) <= 96 * 512) return true;
