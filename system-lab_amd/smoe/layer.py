@@ -483,10 +483,12 @@ class SimpleMoE(nn.Module):
         _C.call("smoe_layer_backward", ctypes.byref(a), main.cuda_stream, side.cuda_stream)
         if gate:
             # logits = x @ w_gate in fp32: the gating linear's gradients
-            x32, dlogits = inter["x"].float(), out["dlogits"]
-            out["dx"] = (out["dx"].float() + dlogits @ self.w_gate.detach().t()).to(torch.bfloat16)
-            out["dw_gate"] = x32.t() @ dlogits
-            main.wait_stream(side)
+            try:
+                x32, dlogits = inter["x"].float(), out["dlogits"]
+                out["dx"] = (out["dx"].float() + dlogits @ self.w_gate.detach().t()).to(torch.bfloat16)
+                out["dw_gate"] = x32.t() @ dlogits
+            finally:  # the side stream still uses scratch, dw1 and dw2: joined also after an error
+                main.wait_stream(side)
         return out
 
     def _side_stream(self, device) -> torch.cuda.Stream:
