@@ -36,6 +36,12 @@ def _install_optimizer_hook():
         _OPT_HOOK.append(register_optimizer_step_post_hook(_count_optimizer_step))
 
 
+def _weight_is(w, s, E: int, N: int, Kd: int) -> bool:
+    """w, s are an fp8 weight [E, N, K] (plain or packed) and its block scales."""
+    return (tuple(w.shape) == (E, N, ops.pad128(Kd))
+            and tuple(s.shape) == (E, ops.nblocks(N), ops.nblocks(Kd)))
+
+
 class _SimpleMoEFunction(torch.autograd.Function):
     """Autograd node of one SimpleMoE forward.  The forward keeps the
     intermediates the fp8 backward needs as saved tensors, so autograd frees
@@ -299,22 +305,24 @@ class SimpleMoE(nn.Module):
             return self._empty_forward(x, logits, save)
         fp8 = self.fp8_weights()
         w1, w1s, w2, w2s = self._gemm
-        H, I, E, K = self.hidden, self.intermediate, self.num_experts, self.top_k
+        K = self.top_k
         ops._check(x, "x", (torch.bfloat16,), 2)
-        T, dev = x.shape[0], x.device
-        if x.shape[1] != H:
-            raise ValueError(f"x must be [T, {H}], got {tuple(x.shape)}")
+        (T, H), dev = x.shape, x.device
         gate = logits if logits is not None else self.w_gate.detach()
         ops._check(gate, "logits", (torch.float32,), 2)
-        if tuple(gate.shape) != ((T if logits is not None else H), E):
-            raise ValueError(f"logits must be [{T}, {E}], got {tuple(gate.shape)}")
         bias = self.router_bias
+        E, I = w1.shape[0], w1.shape[1] // 2
         if bias is not None:
             ops._check(bias, "router_bias", (torch.float32,), 1)
             if bias.numel() != E:
                 raise ValueError("router_bias must have E entries")
-        if w1.device != dev:
-            raise ValueError(f"the weights are on {w1.device}, x on {dev}")
+        if w1.device != dev or w2.device != dev:
+            raise ValueError(f"the weights are on {w1.device} and {w2.device}, x on {dev}")
+        # the native call takes the sizes as numbers: the tensors' own (weights
+        # may be replaced by others), and only where every shape agrees
+        if not (tuple(gate.shape) == ((T if logits is not None else H), E)
+                and _weight_is(w1, w1s, E, 2 * I, H) and _weight_is(w2, w2s, E, H, I)):
+            return self._forward_by_operators(x, logits, save)
         flags = self._layer_flags(w1, w2)
         lib = _C.lib()
         out = torch.empty((T, H), dtype=torch.bfloat16, device=dev)
@@ -345,6 +353,28 @@ class SimpleMoE(nn.Module):
             a.scratch, a.scratch_bytes = buf.data_ptr(), nbytes
         _C.call("smoe_layer_forward", ctypes.byref(a), ops._stream())
         return (out, inter) if save else out
+
+    def _forward_by_operators(self, x, logits, save):
+        """The forward as its single operators, each checking its arguments:
+        for weights whose w2 rows are not as many as x's columns (x padded by
+        the caller, say); other shapes that do not agree are refused there."""
+        w1, w1s, w2, w2s = self._gemm
+        K, rs, e8 = self.top_k, self._row_scale, self._pow2
+        if logits is None:
+            logits = ops.gate_logits(x, self.w_gate.detach(), K)
+        idx, w, row_map, inv_map, counts, off = ops.route_topk_sort(logits, K, self.router_bias)
+        xq, xs = ops.permute_quant_rows(x, inv_map, K, scale=rs)
+        if save:
+            c1 = ops.grouped_gemm_fp8(xq, xs, w1, w1s, off, e8m0=e8)
+            hq, hs, h = ops.swiglu_quant(c1, save_h=True, scale=rs)
+        else:
+            hq, hs = ops.grouped_gemm_fp8_swiglu(xq, xs, w1, w1s, off, scale=rs)
+        y = ops.grouped_gemm_fp8(hq, hs, w2, w2s, off, e8m0=e8)
+        out = ops.unpermute_combine(y, inv_map, w)
+        if not save:
+            return out
+        return out, dict(x=x, logits=logits, topk_idx=idx, topk_w=w, row_map=row_map, inv_map=inv_map,
+                         counts=counts, offsets=off, xq=xq, xs=xs, c1=c1, hq=hq, hs=hs, h=h, y=y, fp8=self._fp8)
 
     def _layer_flags(self, w1, w2) -> int:
         return ((_C.SMOE_LAYER_W1_PACKED if isinstance(w1, ops.PackedWeight) else 0)
@@ -432,6 +462,8 @@ class SimpleMoE(nn.Module):
                 out["dw2"] = dw2_into
             return out
         w1t, w1ts, w2t, w2ts = self.gemm_weights_t(inter.get("fp8"))
+        if not (_weight_is(w1t, w1ts, E, H, 2 * I) and _weight_is(w2t, w2ts, E, I, H)):
+            raise ValueError(f"the weights are not those of {E} experts, hidden {H}, intermediate {I}")
         K, T = self.top_k, inter["x"].shape[0]
         R, dev = T * K, dout.device
         dout = dout.contiguous()

@@ -104,6 +104,32 @@ def test_layer_calls_refuse_what_the_operators_refused(dev):
         m.backward_from(dict(st, c1=st["c1"].float()), x)
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("recipe", ["blockwise", "e8m0"])
+def test_layer_with_replaced_weights(dev, recipe):
+    """Weights of other sizes put into a module run as in a module of those
+    sizes (fewer experts, another width), and x wider than w2's rows as the
+    operators run it (rows padded by the caller to whole 128-column groups)."""
+    print("[replaced]", recipe, flush=True)
+    g = torch.Generator(device=dev).manual_seed(3)
+    small, m = (smoe.SimpleMoE(H, I, E, 2, device=dev, recipe=recipe) for H, I, E in ((512, 256, 4), (512, 512, 8)))
+    small.reset_parameters(g)
+    m.w1.data, m.w2.data, m.w_gate.data = small.w1.data, small.w2.data, small.w_gate.data
+    x, lg = W.tokens(40, 512, device=dev), W.logits(40, 4, device=dev)
+    with torch.no_grad():
+        assert torch.equal(m(x, lg), small(x, lg)) and torch.equal(m(x), small(x))
+        a, b = (q(x, lg, return_intermediates=True)[1] for q in (m, small))
+        for k in ("c1", "hq", "y", "offsets"):
+            assert torch.equal(u8(a[k]), u8(b[k])), k
+    odd = smoe.SimpleMoE(528, 256, 4, 2, device=dev, recipe=recipe)
+    odd.reset_parameters(g)
+    wide = torch.nn.functional.pad(W.tokens(40, 528, device=dev), (0, 640 - 528))
+    with torch.no_grad():
+        out = odd(wide, lg)
+        assert out.shape == (40, 528) and torch.equal(u8(out), u8(odd(wide[:, :528], lg)))
+        assert torch.equal(u8(out), u8(odd(wide, lg, return_intermediates=True)[0]))
+
+
 def test_layer_entry_points_reject():
     lib = _C.lib()
     assert lib.smoe_layer_forward(None, None) == -1 and lib.smoe_layer_backward(None, None, None) == -1

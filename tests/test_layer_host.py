@@ -65,3 +65,54 @@ def test_streams_are_joined_when_the_gate_gradient_fails(host):
     with pytest.raises(RuntimeError):
         m.backward_from(st, torch.zeros(T, H, dtype=torch.bfloat16))
     assert calls[-2] == "smoe_layer_backward" and calls[-1][:2] == ("wait", main)
+
+
+@pytest.mark.parametrize("change", [
+    dict(E=4), dict(I=64), dict(H=128),                       # all weights of another layer
+    dict(w1=(E, 2 * I, 128)), dict(w1=(E - 1, 2 * I, H)),     # one tensor that does not fit the rest
+    dict(w2=(E, H, 256)), dict(w2=(E - 1, H, I))])
+@pytest.mark.parametrize("save", [False, True])
+def test_forward_never_runs_on_weights_of_other_shapes(host, change, save):
+    """The native call takes the sizes as numbers: it is made only with
+    weights of exactly those shapes.  Weights a caller replaced by others run
+    with their own sizes or are refused, as the operators did."""
+    calls, _ = host
+    m = module()
+    set_weights(m, change.get("E", E), change.get("I", I), change.get("H", H))
+    w1, w1s, w2, w2s = m._gemm
+    w1 = torch.zeros(change.get("w1", w1.shape), dtype=torch.uint8)
+    w2 = torch.zeros(change.get("w2", w2.shape), dtype=torch.uint8)
+    m._fp8 = m._gemm = (w1, w1s, w2, w2s)
+    x, logits = torch.zeros(T, H, dtype=torch.bfloat16), torch.zeros(T, E)
+    if change == dict(I=64):  # a consistent layer of another width: runs, with its own sizes
+        with torch.no_grad():
+            out = m(x, logits, return_intermediates=save)
+        if save:
+            assert out[1]["c1"].shape == (T * K, 128) and out[1]["hq"].shape == (T * K, 128)
+        return
+    with pytest.raises(ValueError), torch.no_grad():
+        m(x, logits, return_intermediates=save)
+    assert "smoe_layer_forward" not in calls
+
+
+def test_forward_takes_the_sizes_of_replaced_weights(host):
+    """Experts dropped from all three parameters, as a pruned layer has it."""
+    calls, _ = host
+    m = module()
+    set_weights(m, 4, I, H)
+    with torch.no_grad():
+        _, st = m(torch.zeros(T, H, dtype=torch.bfloat16), torch.zeros(T, 4), return_intermediates=True)
+    assert st["offsets"].shape == (5,) and calls == ["smoe_layer_forward"]
+
+
+@pytest.mark.parametrize("t", range(4))
+def test_backward_never_runs_on_weights_of_other_shapes(host, t):
+    calls, _ = host
+    m = module()
+    st = intermediates(m)
+    bad = list(m._gemm_t)
+    bad[t] = torch.zeros([n - 1 for n in bad[t].shape], dtype=bad[t].dtype)
+    m._gemm_t = tuple(bad)
+    with pytest.raises(ValueError):
+        m.backward_from(st, torch.zeros(T, H, dtype=torch.bfloat16))
+    assert "smoe_layer_backward" not in calls
