@@ -461,6 +461,8 @@ class SimpleMoE(nn.Module):
             if dw2_into is not None:
                 out["dw2"] = dw2_into
             return out
+        if (dw1_into is None or dw2_into is None) and wgrad_dtype not in (torch.float32, torch.bfloat16):
+            raise TypeError("the weight gradient is fp32 or bf16")
         w1t, w1ts, w2t, w2ts = self.gemm_weights_t(inter.get("fp8"))
         if not (_weight_is(w1t, w1ts, E, H, 2 * I) and _weight_is(w2t, w2ts, E, I, H)):
             raise ValueError(f"the weights are not those of {E} experts, hidden {H}, intermediate {I}")

@@ -116,3 +116,9 @@ def test_backward_never_runs_on_weights_of_other_shapes(host, t):
     with pytest.raises(ValueError):
         m.backward_from(st, torch.zeros(T, H, dtype=torch.bfloat16))
     assert "smoe_layer_backward" not in calls
+
+
+def test_backward_refuses_other_gradient_types(host):
+    m = module()
+    with pytest.raises(TypeError):
+        m.backward_from(intermediates(m), torch.zeros(T, H, dtype=torch.bfloat16), wgrad_dtype=torch.float16)
