@@ -312,6 +312,14 @@ int smoe_quantize_pack_weight(const uint16_t* w, int E, int N, int Kdim, uint8_t
                               uint8_t* wp, int scale_mode, void* stream);
 
 /*
+ * Which kernel a grouped GEMM call takes (a host-side query; the result is the
+ * same either way): 0 the 256-row one, else the columns per workgroup (64, 128
+ * or 256) of the one for few rows per expert.  layout: 0 plain weights, 1
+ * packed, 2 packed with power-of-two scales; swiglu: the fused fc1 form, N = 2I.
+ */
+int smoe_grouped_gemm_small_cols(int layout, int swiglu, int E, int R, int N, int Kdim);
+
+/*
  * smoe_grouped_gemm_fp8 on packed weights (smoe_pack_weight_fp8): the same
  * c [R,N] bf16 (bit for bit whenever each 128-wide K block's products sum
  * exactly in fp32; else within the last bf16 bit), from a kernel that loads each wave's weights

@@ -13,6 +13,9 @@ enum class SmallWeights { kPacked, kPlain };
 // the small-row kernel (N = 2I in the fused SwiGLU form).
 bool small_gemm_rows(SmallWeights lay, bool e8m0, bool swiglu, int E, int R, int N, int Kdim);
 
+// Its column tiles are 64 times this many columns wide.
+int small_gemm_cols(bool swiglu, int E, int R, int N);
+
 // Whether the 256-row kernels should skip the empty 16-row blocks of an
 // expert's last tile (kShort): the launch has more than one round of 256 x 256
 // tiles, NT column tiles wide (in one round the fullest tile decides, and the

@@ -23,6 +23,9 @@
 // each.  At most 256 registers and 68 KiB of LDS leave two workgroups per
 // CU, so one tile's start and end hide behind the other's stream.
 //
+// With 65 rows or more and few tiles the workgroup may take 64 rows instead
+// (find_tile decides, see kLowRows).
+//
 // Every wave finds the workgroup's tile by itself (wave scans over the
 // experts' tile counts): no LDS and no barrier before the first load.
 // Tiles are numbered expert by expert and dealt to the XCDs in 8 contiguous
@@ -51,19 +54,36 @@ template <bool kE8>
 constexpr int kTileRows = kE8 ? 128 : 112;
 constexpr int kMaxChunk = 16 * 1024;  // most activation bytes of a chunk
 
+// Tall experts are cut into tiles of kLowRows rows instead of kTileRows while
+// the launch then still has at most two workgroups per CU (kLowMax): its time
+// is that of its tallest tile, a taller loop waits longer per K step (the 64-row
+// loop takes two K steps of activations at once), and the experts' sizes
+// are only known here.  Not where the tall tiles would have a CU each and the
+// low ones not (kCUs): a CU with two tiles streams twice the weights.  us without ->
+// with (fused SwiGLU; the 256-row kernels in brackets), Zipf(1.2) loads: E 128, N
+// 1536, K 2048, 128 rows, packed 29.1 -> 18.8 (32.3); E 96, N 1024, K 4608, 192 rows, plain
+// 68.6 -> 42.9 (64.0); E 16, N 4608, K 3584, 512 rows, packed 79.7 -> 61.1 (83.0);
+// random loads: E 8, N 4096, K 1024, 512 rows, plain 26.2 -> 18.9 (23.0).
+constexpr int kLowRows = 64, kLowMax = 512, kCUs = 256;
+
 struct Tile {
   int row0, rows, e, nt;
 };
 
 // The tile of workgroup bid: false when it is past the last one.  offsets[] is
 // device data the host never sees: whatever it holds, rows stay in [0, R).
+// low: the height of the tiles is chosen here.  An expert's rows are then at
+// most R <= kLowMax * kLowRows, so counts of both heights share a word (64
+// experts' sums stay below 2^16) and need no bound of their own.
 template <int kBM>
 __device__ __forceinline__ bool find_tile(const int32_t* __restrict__ offsets, int E, int R, int NT,
-                                          int mt_bound, int bid, int lane, Tile& t) {
+                                          int mt_bound, bool low, int bid, int lane, Tile& t) {
   auto row_at = [&](int e) { return max(0, min(offsets[min(e, E)], R)); };
+  // tiles of an expert; with low, those of kLowRows rows in the high half
   auto tiles = [&](int e) {
-    const int o0 = row_at(e), o1 = row_at(e + 1);
-    return o1 > o0 ? min((o1 - o0 + kBM - 1) / kBM, mt_bound) : 0;
+    const int n = max(row_at(e + 1) - row_at(e), 0);
+    const int c = min((n + kBM - 1) / kBM, mt_bound);
+    return low ? c | (n + kLowRows - 1) / kLowRows << 16 : c;
   };
   auto scan = [&](int v) {
 #pragma unroll
@@ -77,18 +97,24 @@ __device__ __forceinline__ bool find_tile(const int32_t* __restrict__ offsets, i
   int cnt[kHeld], inc[kHeld];
 #pragma unroll
   for (int i = 0; i < kHeld; ++i) cnt[i] = tiles(i * kWave + lane);
-  int total = 0;
+  int total = 0, total_low = 0;
+  auto add = [&](int v) {
+    total = min(total + (low ? v & 0xffff : v), mt_bound);
+    total_low += (int)((uint32_t)v >> 16);
+  };
 #pragma unroll
   for (int i = 0; i < kHeld; ++i) {
     if (i * kWave < E) {
       inc[i] = scan(cnt[i]);
-      total = min(total + __builtin_amdgcn_readlane(inc[i], kWave - 1), mt_bound);
+      add(__builtin_amdgcn_readlane(inc[i], kWave - 1));
     }
   }
-  for (int b = kHeld * kWave; b < E; b += kWave) {
-    const int v = scan(tiles(b + lane));
-    total = min(total + __builtin_amdgcn_readlane(v, kWave - 1), mt_bound);
-  }
+  for (int b = kHeld * kWave; b < E; b += kWave)
+    add(__builtin_amdgcn_readlane(scan(tiles(b + lane)), kWave - 1));
+  const bool cut = low && total_low * NT <= kLowMax && !(total * NT <= kCUs && total_low * NT > kCUs);
+  const int bm = cut ? kLowRows : kBM;
+  if (cut) total = total_low;
+  auto count = [&](int v) { return low ? (cut ? (int)((uint32_t)v >> 16) : v & 0xffff) : v; };
   // 8 contiguous ranges of tiles, one per XCD; an expert's row tiles of one
   // column tile are neighbours, so its weights are read from memory once
   const int all = total * NT;
@@ -112,18 +138,18 @@ __device__ __forceinline__ bool find_tile(const int32_t* __restrict__ offsets, i
   bool found = false;
 #pragma unroll
   for (int i = 0; i < kHeld; ++i)
-    if (!found && i * kWave < E) found = take(i * kWave, cnt[i], inc[i]);
+    if (!found && i * kWave < E) found = take(i * kWave, count(cnt[i]), count(inc[i]));
   for (int b = kHeld * kWave; b < E && !found; b += kWave) {
-    const int c = tiles(b + lane);
+    const int c = count(tiles(b + lane));
     found = take(b, c, scan(c));
   }
   if (!found || t.e >= E) return false;
   const int q = tl - first * NT;
   t.nt = q / nt_e;
-  // the expert's n rows in nt_e = ceil(n / kBM) tiles of equal height, a
-  // multiple of 16: at most kBM, so the last one is never empty
+  // the expert's n rows in nt_e = ceil(n / bm) tiles of equal height, a
+  // multiple of 16: at most bm, so the last one is never empty
   const int o0 = row_at(t.e), o1 = row_at(t.e + 1);
-  const int h = min(((o1 - o0 + nt_e - 1) / nt_e + 15) & ~15, kBM);
+  const int h = min(((o1 - o0 + nt_e - 1) / nt_e + 15) & ~15, bm);
   t.row0 = o0 + (q - t.nt * nt_e) * h;
   t.rows = min(h, o1 - t.row0);
   return t.rows > 0;
@@ -293,7 +319,8 @@ template <SmallWeights kLay, bool kE8, bool kSwiGLU, int kCB>
 __global__ __launch_bounds__(kThreads, 2) void gemm_small_kernel(
     const uint8_t* __restrict__ a, const float* __restrict__ as, const uint8_t* __restrict__ b,
     const float* __restrict__ bs, const int32_t* __restrict__ offsets, int E, int R, int N, int Kd,
-    int mt_bound, uint16_t* __restrict__ c, uint8_t* __restrict__ hq, float* __restrict__ hs) {
+    int mt_bound, bool low, uint16_t* __restrict__ c, uint8_t* __restrict__ hq,
+    float* __restrict__ hs) {
   static_assert(!kSwiGLU || kCB == 4, "fused SwiGLU pairs 128 gate with 128 up columns");
   constexpr int kBN = 64 * kCB, kCPitch = kBN * 2 + 16, kBM = kTileRows<kE8>;
   constexpr int kLoop = 2 * kMaxChunk + 2 * kThreads * 4;
@@ -304,7 +331,7 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_small_kernel(
   const int I = N / 2;
   const int NT = kSwiGLU ? I / kGroup : (N + kBN - 1) / kBN;
   Tile t;
-  if (!find_tile<kBM>(offsets, E, R, NT, mt_bound, blockIdx.x, lane, t)) return;  // the whole workgroup leaves
+  if (!find_tile<kBM>(offsets, E, R, NT, mt_bound, low, blockIdx.x, lane, t)) return;  // the whole workgroup leaves
   const int e = t.e, row0 = t.row0, rows = t.rows, nt = t.nt;
   const int n0 = nt * kBN, ksb = Kd / kBK, NB = (N + kGroup - 1) / kGroup;
 
@@ -409,11 +436,27 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_small_kernel(
 // and without the epilogue K < 1024: E8M0 to 1024 rows 1.01 - 1.48 (N 2048, K 768,
 // E 128: 512 rows 213 -> 195; at 2048 rows and N 256 0.86), K 512 to 512 rows 1.03 -
 // 1.53 (at 1024 rows 0.98).
+//
+// 4. Between half a round and one round of 256 x 256 tiles if every expert has
+// one (128 < E * N/256 <= 256) the 256-row kernels stream at their best and this
+// one gains least.  45 shapes (E 8 - 64, K 1408 - 7168), means and the
+// worst, fused SwiGLU / without, random then Zipf(1.2) loads:
+//   plain, up to 192 tiles: 56 rows 1.27 (1.20) / 1.28 (1.24), 1.35 (0.95) / 1.22 (0.91); 72
+//     rows 0.87 (0.84) / 80 rows 0.88 (0.84).  Above 192: 48 rows 1.16 (0.88) / 1.19 (0.90),
+//     1.05 (0.94) / 0.94 (0.86); 56 rows 0.90 (0.87) / 0.93 (0.89), 1.03 (0.91) / 0.90 (0.85)
+//   packed, K > 3072: 64 rows 1.12 (0.92) / 1.13 (0.95), 1.22 (0.98) / 1.16 (0.95); 72 rows
+//     0.96 (0.88) with SwiGLU; E8M0 64 rows 1.11 (0.95) / 1.11 (0.96), 72 rows 0.98 (0.95)
+//     with SwiGLU.  K <= 3072: as in 1.
 bool small_gemm_rows(SmallWeights lay, bool e8m0, bool swiglu, int E, int R, int N, int Kdim) {
   const bool packed = lay == SmallWeights::kPacked;
-  const long long one_tile = !packed ? 80
-                             : e8m0  ? (Kdim <= 4096 ? 112 : Kdim <= 8192 ? 80 : 64)
-                                     : (Kdim <= 8192 ? 112 : 80);
+  long long one_tile = !packed ? 80
+                       : e8m0  ? (Kdim <= 4096 ? 112 : Kdim <= 8192 ? 80 : 64)
+                               : (Kdim <= 8192 ? 112 : 80);
+  const long long t256 = (N + 255) / 256 * (long long)E;
+  if (t256 > 128 && t256 <= 256) {
+    if (!packed) one_tile = t256 <= 192 ? 56 : 48;
+    else if (Kdim > 3072) one_tile = 64;
+  }
   auto to = [&](long long rows) { return R <= rows * E; };
   if (to(one_tile)) return true;
   if ((packed || !swiglu) && (2LL * R + 256LL * E) * ((N + 255) / 256) <= 96 * 512) return true;
@@ -421,6 +464,28 @@ bool small_gemm_rows(SmallWeights lay, bool e8m0, bool swiglu, int E, int R, int
   if (!swiglu) return Kdim < 1024 && to(e8m0 ? 1024 : 512);
   if (Kdim <= (e8m0 ? 2048 : 1536)) return to(8192);
   return Kdim <= (e8m0 ? 3072 : 2048) && R >= 256LL * E && to(1024);
+}
+
+// Column tiles of 64 * small_gemm_cols columns: 4, or without SwiGLU 2 or 1.
+// Narrower while the launch has fewer than two workgroups per CU, because few
+// workgroups stream too little.  Not so from 16 rows per expert on (8 above
+// 192 tiles) where 256 columns make half a round to a round of workgroups, one
+// per expert and column tile: narrower ones are then two or four rounds that
+// each read the activations again.  45 shapes (as in 4 above), former width -> this
+// one, means against the 256-row kernels, random and Zipf(1.2) loads: plain 32 rows
+// 1.26 -> 1.33, 1.08 -> 1.25; packed 48 rows 1.24 -> 1.35, 1.03 -> 1.18; E8M0 56 rows 1.13 ->
+// 1.23, 1.04 -> 1.17.  Above 64 rows, two tiles an expert, 128 columns: packed 80 rows
+// 1.07 -> 1.15, 0.95 -> 1.12.  At fewer rows random loads prefer the narrow ones (up to
+// 192 tiles, plain 10 rows 1.51 against 1.41), and at 256 tiles, 512 workgroups of
+// 128 columns, they stay ahead (E 32, N 2048, packed 48 rows 1.25 against 1.09).
+int small_gemm_cols(bool swiglu, int E, int R, int N) {
+  if (swiglu) return 4;
+  const long long t256 = (N + 255) / 256 * (long long)E;
+  if (t256 > 128 && t256 < 256 && R > (t256 <= 192 ? 16LL : 8LL) * E) return R > (long long)small::kLowRows * E ? 2 : 4;
+  const long long live = E < R ? E : R;
+  int cb = 4;
+  while (cb > 1 && live * (long long)((N + 64 * cb - 1) / (64 * cb)) < 512) cb >>= 1;
+  return cb;
 }
 
 int small_gemm_launch(SmallWeights lay, bool e8m0, const uint8_t* a, const float* as,
@@ -432,19 +497,24 @@ int small_gemm_launch(SmallWeights lay, bool e8m0, const uint8_t* a, const float
   const int bm = e8m0 ? small::kTileRows<true> : small::kTileRows<false>;
   const long long mt = live + ((long long)R + bm - 1) / bm;
   const bool swiglu = hq != nullptr;
-  int cb = 4;
-  if (!swiglu) {
-    // columns per workgroup: narrower while the launch has fewer than two
-    // workgroups per CU
-    while (cb > 1 && live * (long long)((N + 64 * cb - 1) / (64 * cb)) < 512) cb >>= 1;
-  }
+  const int cb = small_gemm_cols(swiglu, E, R, N);
   const long long NT = swiglu ? N / 2 / kGroup : (N + 64 * cb - 1) / (64 * cb);
-  const long long nblk = (mt * NT + 7) / 8 * 8;
+  // the kernel may take kLowRows rows per tile where that can fit kLowMax: the
+  // grid then holds kLowMax workgroups of them, or all there can be
+  const long long cut = ((long long)R + small::kLowRows - 1) / small::kLowRows;
+  const bool low = R > small::kLowRows && cut * NT <= small::kLowMax;
+  long long bound = mt;
+  if (low) {
+    const long long fit = (small::kLowMax + NT - 1) / NT;
+    bound = live + cut < fit ? live + cut : fit;
+    if (bound < mt) bound = mt;
+  }
+  const long long nblk = (bound * NT + 7) / 8 * 8;
   if (nblk > 0x7fffffffLL) return SMOE_EINVAL_DIM;
 #define SMOE_SG(LAY, E8, SW, CB)                                                                \
   small::gemm_small_kernel<SmallWeights::LAY, E8, SW, CB>                                        \
       <<<dim3((unsigned)nblk), dim3(small::kThreads), 0, stream>>>(a, as, b, bs, offsets, E, R, \
-                                                                   N, Kdim, (int)mt, c, hq, hs)
+                                                                   N, Kdim, (int)bound, low, c, hq, hs)
 #define SMOE_SG_CB(LAY, E8)                    \
   do {                                         \
     if (swiglu) SMOE_SG(LAY, E8, true, 4);     \
@@ -461,3 +531,11 @@ int small_gemm_launch(SmallWeights lay, bool e8m0, const uint8_t* a, const float
 }
 
 }  // namespace smoe
+
+extern "C" int smoe_grouped_gemm_small_cols(int layout, int swiglu, int E, int R, int N, int Kdim) {
+  using namespace smoe;
+  if (E <= 0 || R <= 0 || N <= 0 || Kdim <= 0 || layout < 0 || layout > 2) return 0;
+  const SmallWeights lay = layout ? SmallWeights::kPacked : SmallWeights::kPlain;
+  if (!small_gemm_rows(lay, layout == 2, swiglu != 0, E, R, N, Kdim)) return 0;
+  return 64 * small_gemm_cols(swiglu != 0, E, R, N);
+}

@@ -48,6 +48,7 @@ SIGNATURES = {
                                              P, P]),
     "smoe_quantize_pack_weight": (c_int, [P, c_int, c_int, c_int, P, P, P, c_int, P]),
     "smoe_transpose_pack_fp8": (c_int, [P, P, c_int, c_int, c_int, P, P, P]),
+    "smoe_grouped_gemm_small_cols": (c_int, [c_int] * 6),
     "smoe_pack_weight_fp8": (c_int, [P, c_int, c_int, c_int, P, P]),
     "smoe_grouped_gemm_fp8_packed": (c_int, [P, P, P, P, P, c_int, c_int, c_int, c_int, P, P]),
     "smoe_grouped_gemm_fp8_packed_e8m0": (c_int, [P, P, P, P, P, c_int, c_int, c_int, c_int, P, P]),

@@ -10,7 +10,7 @@ import pytest
 import torch
 
 from oracle import smoe_oracle as O
-from smoe import ops
+from smoe import _C, ops
 from smoe import workloads as W
 
 
@@ -20,11 +20,19 @@ def tiles(R, NT, offsets, BM):
     """(expert, first row, rows, column tile) of every workgroup that works."""
     E = len(offsets) - 1
     offsets = np.clip(offsets, 0, R)
+    n = [max(0, int(offsets[e + 1]) - int(offsets[e])) for e in range(E)]
     bound = min(E, R) + -(-R // BM)
-    cnt = [min(-(-max(0, int(offsets[e + 1]) - int(offsets[e])) // BM), bound) for e in range(E)]
+    cut64 = -(-R // 64)
+    low = R > 64 and cut64 * NT <= 512  # 64-row tiles, if they all run at once
+    if low:
+        bound = max(bound, min(min(E, R) + cut64, -(-512 // NT)))
+    cnt = [min(-(-m // BM), bound) for m in n]
     total = 0
     for b in range(0, E, 64):
         total = min(total + sum(cnt[b:b + 64]), bound)
+    cnt64 = [-(-m // 64) for m in n]
+    if low and sum(cnt64) * NT <= 512 and not (total * NT <= 256 < sum(cnt64) * NT):
+        BM, cnt, total = 64, cnt64, sum(cnt64)
     out, n = [], total * NT
     chunk = (n + 7) // 8
     for bid in range((bound * NT + 7) // 8 * 8):
@@ -35,6 +43,8 @@ def tiles(R, NT, offsets, BM):
         while e < E and first + cnt[e] <= mt:
             first += cnt[e]
             e += 1
+        if e == E:
+            continue
         q = tl - first * NT
         nt = q // cnt[e]
         o0, o1 = int(offsets[e]), int(offsets[e + 1])
@@ -71,6 +81,63 @@ def test_tiles_stay_in_range_for_malformed_offsets():
         off = int(rng.integers(-300, 300)) + np.concatenate([[0], np.cumsum(rng.integers(-300, 900, E))])
         for _, row0, rows, _ in tiles(R, 2, off, 112):
             assert 0 <= row0 and row0 + rows <= R and rows <= 112
+
+
+# loads on the edges of the choice of 64-row tiles: counts, N of the fused
+# SwiGLU form (128 columns a tile), tile rows chosen
+CUT = [
+    ([65] * 3, 256, 64),
+    ([129] * 50, 1024, 112),        # 64-row tiles: 600 workgroups, past 512; 400 of 112 rows
+    ([129] * 42 + [1], 1024, 64),   # 127 x 4 workgroups
+    ([128] * 64, 1024, 64),         # 128 x 4: 512 exactly
+    ([128] * 63 + [129], 1024, 112),
+    ([112] * 16, 4096, 112),        # 16 x 16: a CU each; the low tiles would be 512
+    ([113] + [112] * 15, 4096, 64),
+    ([113, 113] + [40] * 13, 4096, 64),
+    ([64] * 16, 4096, 64), ([2000, 0, 1, 17], 1024, 64),
+    ([0, 700] + [3] * 300, 256, 64),
+]
+
+
+def test_tile_height_at_its_edges():
+    for counts, N, rows in CUT:
+        t = tiles(sum(counts), N // 256, np.concatenate([[0], np.cumsum(counts)]), 112)
+        assert max(r for _, _, r, _ in t) <= rows, (counts, rows)
+        seen = np.zeros((sum(counts), N // 256), int)
+        for _, row0, r, nt in t:
+            seen[row0:row0 + r, nt] += 1
+        assert (seen == 1).all()
+        assert rows == 64 or max(r for _, _, r, _ in t) > 64
+
+
+def small_cols(form, swiglu, E, R, N, K):
+    """Columns per workgroup of the small-row kernel, 0: the 256-row one."""
+    return _C.lib().smoe_grouped_gemm_small_cols({"plain": 0, "packed": 1, "e8m0": 2}[form], swiglu, E, R, N, K)
+
+
+@pytest.mark.parametrize("form,swiglu,E,N,K,line", [
+    ("plain", True, 16, 2560, 1408, 56),     # 160 tiles of 256 x 256: up to three quarters of a round
+    ("plain", False, 24, 2560, 4480, 48),    # 240
+    ("plain", True, 32, 2048, 7168, 48),     # 256: a whole round
+    ("packed", False, 24, 2560, 7168, 64), ("e8m0", True, 16, 2560, 4480, 64),
+    ("plain", True, 8, 4096, 1024, 80),      # 128: half a round
+    ("plain", False, 32, 4096, 7168, 80),    # 512
+    ("packed", False, 32, 4096, 7168, 112), ("packed", False, 24, 2560, 2048, 112),
+    ("e8m0", False, 32, 5760, 2944, 112),
+])
+def test_lines_between_the_kernels(form, swiglu, E, N, K, line):
+    """Few rows per expert under skewed loads lost to the 256-row kernels where
+    those have nearly a round of tiles: the lines are lower there."""
+    assert small_cols(form, swiglu, E, E * line, N, K) > 0
+    assert small_cols(form, swiglu, E, E * line + 1, N, K) == 0
+
+
+@pytest.mark.parametrize("E,N,rows,cols", [
+    (24, 2560, 8, 64), (24, 2560, 9, 256), (24, 2560, 64, 256), (24, 2560, 65, 128),
+    (16, 2560, 16, 64), (16, 2560, 17, 256), (32, 2048, 40, 128), (8, 4096, 40, 64), (128, 2048, 40, 256),
+])
+def test_columns_per_workgroup(E, N, rows, cols):
+    assert small_cols("packed", False, E, E * rows, N, 2048) == cols
 
 
 # ------------------------------------------------------------------- GPU
@@ -148,6 +215,27 @@ def test_small_rows_equal_the_256_row_kernels(dev, counts, N, K, form):
             # bf16 rounds to 2^-9 of a value, about 1.4e-3 on average
             d = np.abs(got - ref)
             assert d.max() <= 1e-2 * np.abs(ref).max() and d.mean() <= 2e-3 * np.abs(ref).mean()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("counts,N,_", CUT)
+@pytest.mark.parametrize("form", ["plain", "packed", "e8m0"])
+def test_tile_heights_equal_the_256_row_kernels(dev, counts, N, _, form):
+    """Both heights of the small-row kernel's tiles, against the 256-row ones."""
+    print("[cut]", form, len(counts), N, flush=True)
+    E, n, K, e8m0 = len(counts), sum(counts), 1536, form == "e8m0"
+    big = n + 8193 * E
+    assert small_cols(form, True, E, big, N, K) == 0
+    if form == "plain" and not small_cols(form, True, E, n, N, K):
+        pytest.skip("above the line of plain weights")
+    assert small_cols(form, True, E, n, N, K) == 256
+    scale = "pow2" if e8m0 else "amax"
+    off = W.offsets_from_counts(counts, dev)
+    xq, xs = ops.quant_rows(W.tokens(n, K, device=dev, seed=n), scale=scale)
+    wq, ws = ops.quantize_weight_blockwise(W.weights(E, N, K, device=dev, seed=N), scale=scale)
+    w = wq if form == "plain" else ops.pack_weight_fp8(wq)
+    for a, b in zip(run(xq, xs, w, ws, off, n, e8m0, True, N), run(xq, xs, w, ws, off, big, e8m0, True, N)):
+        assert torch.equal(a, b)
 
 
 @pytest.mark.gpu
