@@ -397,8 +397,10 @@ __global__ __launch_bounds__(C::kThreads, 1) void grouped_gemm_fp8_kernel(
 using GemmCfg = SMOE_GEMM_CFG;
 
 // The instantiation of one call: the scale staging by K, the short tiles by
-// load.  The SwiGLU form with staged scales has no registers left for them (5
-// spills: N 4096, K 7168, 500 rows per expert 612 -> 680 us).
+// load.  The SwiGLU form has no registers left for them: 5 spills with staged
+// scales (N 4096, K 7168, 500 rows per expert 612 -> 680 us), 4 without, where it
+// lost 2 - 8% at every load from 90 to 1024 rows (N 5888, K 2944, E 32).  The plain
+// form with staged scales spills one and gains all the same (above).
 #define SMOE_PLAIN_K(SW, CH, SH, W, WS, ...)                                                 \
   grouped_gemm_fp8_kernel<C, SW, CH, SH>                                                     \
       <<<dim3((unsigned)nblk), dim3(C::kThreads), 0, (hipStream_t)stream>>>(                 \
@@ -406,9 +408,9 @@ using GemmCfg = SMOE_GEMM_CFG;
 #define SMOE_PLAIN(SW, W, WS, ...)                                      \
   do {                                                                  \
     const bool chunk = Kdim % (kBK * 4) == 0;                           \
-    const bool cut = !(SW && chunk) && short_tiles(E, R, NT, 256, 256, 1024); \
+    const bool cut = !SW && short_tiles(E, R, NT, 256, 256, 1024);      \
     if (cut && chunk) SMOE_PLAIN_K(SW, true, !SW, W, WS, __VA_ARGS__);  \
-    else if (cut) SMOE_PLAIN_K(SW, false, true, W, WS, __VA_ARGS__);    \
+    else if (cut) SMOE_PLAIN_K(SW, false, !SW, W, WS, __VA_ARGS__);     \
     else if (chunk) SMOE_PLAIN_K(SW, true, false, W, WS, __VA_ARGS__);  \
     else SMOE_PLAIN_K(SW, false, false, W, WS, __VA_ARGS__);            \
     SMOE_RETURN_LAUNCH();                                               \
