@@ -75,11 +75,14 @@ __device__ __forceinline__ int e8m0_of(float s) { return (__float_as_uint(s) >> 
 // with 256 of them the compiler's own MFMA form needs a spare quad for a
 // fresh destination, which the accumulation file does not have, and it then
 // moves accumulators through the architectural registers every step.
-// Hazards: the accumulators are written only by these MFMAs (an accumulator
-// is reused 64 MFMAs later); a row block's first MFMA starts with two wait
-// states after the VALU that may have just written its scale operands; the
-// epilogue waits out the last MFMA with explicit s_nops.  Operand loads are waited for by the compiler, which sees
-// the asm's register uses.
+// Hazards: the accumulators are written only by these MFMAs, and one is used
+// again a K step later, that is after 4 MFMAs per row block of the step: 64 in
+// the full loop, 16 in the shortest (4 row blocks), where in-order issue alone
+// puts more than an MFMA's latency between them; a row block's first MFMA
+// starts with two wait states after the VALU that may have just written its
+// scale operands; the epilogue waits out the last MFMA with explicit s_nops.
+// Operand loads are waited for by the compiler, which sees the asm's register
+// uses.
 template <bool kNop>
 __device__ __forceinline__ void mfma_scale_acc(v4f& acc, const v8i& a, const v8i& b, int sa,
                                                int sb) {
@@ -295,13 +298,15 @@ __global__ __launch_bounds__(kThreads, 1) void grouped_gemm_fp8_e8m0_kernel(
 
   // ---- one K step: weights of step kb in cur, those of step kb+3 loaded
   // into nxt (the buffer step kb-1 used).  The activation DMAs of a step go
-  // out before its first 8 row blocks and the weight loads before the last
-  // 8.  The compiler waits for cur itself, counting only its own loads: the
-  // 16 loads it sees after cur (steps kb-2 and kb-1) make it wait until at
-  // most 16 memory operations are outstanding, which with the DMAs in the
-  // same in-order counter retires everything up to step kb-2 (stage kb+1
-  // and the weights of step kb+1, both needed within the next step) and
-  // leaves step kb-1's loads in flight.  Past the last step the loads repeat
+  // out before the first half of its row blocks and the weight loads before
+  // the second half: one before each of 16 blocks, two of 8, four of 4; 16 a
+  // step in each loop, in this order.  The compiler waits for cur itself, at
+  // the asm below and so before the step's first load, counting only its own
+  // loads: the 16 loads it sees after cur (steps kb-2 and kb-1) make it wait
+  // until at most 16 memory operations are outstanding, which with the DMAs
+  // in the same in-order counter retires everything up to step kb-2 (stage
+  // kb+1 and the weights of step kb+1, both needed within the next step) and
+  // leaves step kb-1's 16 in flight.  Past the last step the loads repeat
   // step ksb-1's data into buffers and stages no later step reads.
   auto step = [&](auto m, int kb, WBuf& cur, WBuf& nxt, bool tail) __attribute__((always_inline)) {
     constexpr int kM = decltype(m)::value;  // row blocks with rows: 16, 8 or 4
@@ -375,7 +380,9 @@ __global__ __launch_bounds__(kThreads, 1) void grouped_gemm_fp8_e8m0_kernel(
   // skipped.  us without -> with: E 32, N 5760, K 2944 263 -> 244 (312 rows per
   // expert), 354 -> 334 (512); N 4096, K 7168 303 -> 297 (250), 1660 -> 1612 (2048); E
   // 128, N 1536, K 2048 173 -> 168 (256), 471 -> 461 (1024); between 128 and 256 rows,
-  // where few tiles are short, up to 3% slower.
+  // where few tiles are short, up to 3% slower.  Fused SwiGLU of long K gains to
+  // 320 rows (1.00 - 1.11) and gives up to 3% from 400 on (E 96, N 1024, K 4608); the
+  // form without it spills one register.
   if (!kShort || rows > 128) k_loop(std::integral_constant<int, kRB>{});
   else if (rows > 64) k_loop(std::integral_constant<int, 8>{});
   else k_loop(std::integral_constant<int, 4>{});

@@ -49,7 +49,8 @@ namespace small {
 
 constexpr int kThreads = 256, kWaves = 4;
 // Most rows of a tile: what the registers hold beside two K steps of weights
-// (128 accumulators a lane, or 112 and the products the scales multiply).
+// (128 accumulators a lane, which spills two registers, or 112 and the
+// products the scales multiply).
 template <bool kE8>
 constexpr int kTileRows = kE8 ? 128 : 112;
 constexpr int kMaxChunk = 16 * 1024;  // most activation bytes of a chunk
