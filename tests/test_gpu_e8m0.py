@@ -324,9 +324,9 @@ def _pow2_gemm_operands(dev, counts, N, Kd, seed):
 
 
 def _check_e8m0_gemm(dev, off, xq, xs, wq, ws, rows=None):
-    """E8M0 kernel against the packed kernel on the same operands (the
-    plain kernel where K is not a multiple of 512), within one bf16 ulp and
-    nearly all equal, and against the float64 oracle on the given rows (all
+    """The E8M0 GEMM against the packed one on the same operands (the plain
+    one where K is not a multiple of 512; the small shapes run on the
+    small-row kernel), within one bf16 ulp and nearly all equal, and against the float64 oracle on the given rows (all
     rows by default) at the GEMM bar."""
     wp = ops.pack_weight_fp8(wq)
     got = ops.grouped_gemm_fp8(xq, xs, wp, ws, off, e8m0=True)

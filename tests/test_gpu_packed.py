@@ -1,8 +1,10 @@
 """Packed-weight grouped GEMM (smoe_pack_weight_fp8,
 smoe_grouped_gemm_fp8_packed[_swiglu]): the packed layout byte by byte, and
-the packed kernels held bit-identical to the plain ones (which the oracle
-pins: tests/test_gpu_parity.py) over ragged, empty and skewed experts, tile
-edges and the config-4 shape.  The operands are quantised N(0,1) activations
+the GEMMs on packed weights held bit-identical to those on plain ones (which
+the oracle pins: tests/test_gpu_parity.py) over ragged, empty and skewed
+experts, tile edges and the config-4 shape.  The small shapes run on the
+small-row kernel in both layouts; tests/test_gpu_tile_edges.py has the edges
+on the 256-row kernels.  The operands are quantised N(0,1) activations
 and N(0,0.02) weights, for which each K block's products sum without rounding
 in the MFMA, so the kernels' different K orders cannot show; for operands
 spanning the whole e4m3 range they can, in the last bf16 bit

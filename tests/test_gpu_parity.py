@@ -4,7 +4,11 @@
 Bars: bit-exact for router ids/weights, sort maps, fp8 bytes and scales,
 SwiGLU requant (given the same input) and combine; grouped-GEMM outputs
 within max|d|/max|ref| <= 1e-2 and mean|d|/mean|ref| <= 1e-3 against the
-float64 oracle rounded to bf16 (the reference path's output dtype)."""
+float64 oracle rounded to bf16 (the reference path's output dtype).
+
+GEMM calls of few rows per expert or few tiles run on the small-row kernel,
+as most of the small shapes here do; tests/test_gpu_tile_edges.py has the edge
+cases on the 256-row kernels as well, and pins which shape takes which."""
 import os
 import sys
 
@@ -468,7 +472,7 @@ def _run_gemm(dev, xq, xs, wq, ws, off):
 def test_gemm_layout_one_hot(dev, Kd):
     """Structured operands expose any row/column/K permutation in the MFMA
     fragment or output layout: x[r] = e_(r mod Kd), w[n] = e_n (Kd = 512 also
-    runs the packed-weight kernel)."""
+    runs on packed weights)."""
     say("gemm one-hot layout", Kd)
     R, N, E = 300, 256, 1
     xq = np.zeros((R, Kd), np.uint8)
@@ -518,8 +522,8 @@ def test_gemm_skewed_experts(dev, counts, N, Kd):
 
 
 def test_gemm_max_experts(dev):
-    """E = 1024 (the maximum): the per-workgroup expert scan covers two
-    experts per thread, many experts own no rows, the rest own 1..300."""
+    """E = 1024 (the maximum): the tile search covers 16 experts per lane (the
+    small-row kernel), many experts own no rows, the rest own 1..300."""
     say("gemm 1024 experts")
     rng = np.random.default_rng(1024)
     E, N, Kd = 1024, 256, 256
@@ -534,8 +538,8 @@ def test_gemm_max_experts(dev):
 
 
 def test_gemm_max_kdim(dev):
-    """Kdim = 65536 (the maximum): 512 K blocks, so the tile's weight-scale
-    table in LDS is at its largest."""
+    """Kdim = 65536 (the maximum): 512 K blocks, eight windows of weight scales
+    in the small-row kernel."""
     say("gemm Kdim 65536")
     rng = np.random.default_rng(65536)
     counts = [3, 130]

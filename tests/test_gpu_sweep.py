@@ -7,7 +7,8 @@ nobody thought of are covered too.  Each case is small enough for the
 float64 oracle to finish in well under a second:
 - the router and the expert sort: ids, weights and maps bit-exact;
 - the grouped GEMM, plain, packed and E8M0 (where the shape allows each):
-  within the GEMM bar of the oracle on every row;
+  within the GEMM bar of the oracle on every row (so few tiles run on the
+  small-row kernel; tests/test_gpu_tile_edges.py draws for both kernels);
 - the variable-K weight-gradient GEMM, C3 and E8M0 operands: within the GEMM
   bar, and zero for experts with no rows;
 - the byte-moving stages (permute + quantise, SwiGLU + quantise, the column

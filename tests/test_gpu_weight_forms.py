@@ -13,7 +13,7 @@ u8 = lambda t: t.contiguous().view(torch.uint8)
 
 
 @pytest.mark.parametrize("E,N,K", [(2, 256, 512), (3, 144, 1024), (1, 16, 528), (2, 1536, 2048), (1, 5760, 2880),
-                                   (2, 520 // 8 * 8 - 8, 656)])
+                                   (2, 512, 656)])
 @pytest.mark.parametrize("scale", ["amax", "pow2"])
 def test_one_launch_forms(dev, E, N, K, scale):
     print("[weights]", E, N, K, scale, flush=True)
