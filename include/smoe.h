@@ -190,9 +190,11 @@ int smoe_dispatch_quant(const uint16_t* x, const int32_t* topk_idx, int T, int H
 /*
  * Router, expert sort and permute + 1x128 quantisation of one batch: the
  * outputs of smoe_route_topk_sort then smoe_permute_quant_ex, byte for byte;
- * batches of up to 256 tokens and 2048 pairs in one or two launches.  With
- * logits NULL the logits are x . w_gate [H,E] f32 (fp32 products of the bf16
- * tokens, summed in fp32), for the batches smoe_gate_fused_ok accepts.
+ * batches of up to 256 tokens and 2048 pairs in one or two launches from
+ * logits.  With logits NULL the logits are x . w_gate [H,E] f32 (fp32 products
+ * of the bf16 tokens, summed in fp32), for the batches smoe_gate_fused_ok
+ * accepts, with one more launch.  T decides into how many slices of H a sum is
+ * cut, so a token's logits differ in their last bits between batch sizes.
  * ws: smoe_route_dispatch_workspace_size bytes, status word first.
  * smoe_gate_logits writes the same logits [T,E] f32 (ws as above; its status
  * word is left alone).

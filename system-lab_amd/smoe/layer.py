@@ -143,6 +143,13 @@ class SimpleMoE(nn.Module):
     (``loss.backward()`` fills w1.grad, w2.grad, w_gate.grad and x.grad).
     Without autograd it is the inference path: SwiGLU and its requantisation
     run in the fc1 epilogue and nothing is saved.
+
+    Without ``logits`` they are x @ w_gate in fp32, for small bf16 batches by
+    the layer's own kernel (``ops.gate_fused_ok``), else by a library product.
+    The order of those sums depends on the batch size, so a token's logits can
+    differ in their last bits between batches (and with them, where two experts
+    are that close, its experts); for one batch they are the same with and
+    without autograd.
     """
 
     def __init__(self, hidden: int, intermediate: int, num_experts: int, top_k: int,
