@@ -547,7 +547,9 @@ extern "C" int smoe_quant_cols_ld(int R, int E) {
   return ld > 0x7fffffffLL ? 0 : (int)ld;
 }
 
-int smoe::quant_cols_128x1(const uint16_t* x, const int32_t* gather, int gather_div, int R, int C, const int32_t* offsets, int E, int ld, uint8_t* xTq, float* xTs, int32_t* pad, bool make_pad, int col_scale, void* stream) {
+int smoe::quant_cols_128x1(const uint16_t* x, const int32_t* gather, int gather_div, int R, int C,
+                           const int32_t* offsets, int E, int ld, uint8_t* xTq, float* xTs,
+                           int32_t* pad, bool make_pad, int col_scale, void* stream) {
   if (R <= 0 || C <= 0) return SMOE_EINVAL_DIM;
   if (col_scale != SMOE_COLSCALE_FP32 && col_scale != SMOE_COLSCALE_POW2) return SMOE_EINVAL_MODE;
   if (gather && gather_div <= 0) return SMOE_EINVAL_DIM;
@@ -573,7 +575,9 @@ int smoe::quant_cols_128x1(const uint16_t* x, const int32_t* gather, int gather_
   SMOE_RETURN_LAUNCH();
 }
 
-int smoe::quant_rows_cols(const uint16_t* x, int R, int C, const int32_t* offsets, int E, int ld, uint8_t* xq, float* xs, uint8_t* xTq, float* xTs, int32_t* pad, bool make_pad, int col_scale, void* stream) {
+int smoe::quant_rows_cols(const uint16_t* x, int R, int C, const int32_t* offsets, int E, int ld,
+                          uint8_t* xq, float* xs, uint8_t* xTq, float* xTs, int32_t* pad,
+                          bool make_pad, int col_scale, void* stream) {
   if (R <= 0 || C <= 0) return SMOE_EINVAL_DIM;
   if (col_scale & ~(SMOE_COLSCALE_POW2 | SMOE_ROWSCALE_POW2)) return SMOE_EINVAL_MODE;
   const bool cp2 = col_scale & SMOE_COLSCALE_POW2, rp2 = col_scale & SMOE_ROWSCALE_POW2;
@@ -599,7 +603,10 @@ int smoe::quant_rows_cols(const uint16_t* x, int R, int C, const int32_t* offset
   SMOE_RETURN_LAUNCH();
 }
 
-int smoe::swiglu_bwd_quant(const uint16_t* c1, const uint16_t* dh, int R, int I, const int32_t* offsets, int E, int ld, uint8_t* dcq, float* dcs, uint8_t* dcTq, float* dcTs, int32_t* pad, bool make_pad, uint16_t* dc1, int col_scale, void* stream) {
+int smoe::swiglu_bwd_quant(const uint16_t* c1, const uint16_t* dh, int R, int I,
+                           const int32_t* offsets, int E, int ld, uint8_t* dcq, float* dcs,
+                           uint8_t* dcTq, float* dcTs, int32_t* pad, bool make_pad, uint16_t* dc1,
+                           int col_scale, void* stream) {
   if (R <= 0 || I <= 0) return SMOE_EINVAL_DIM;
   if (col_scale & ~(SMOE_COLSCALE_POW2 | SMOE_ROWSCALE_POW2)) return SMOE_EINVAL_MODE;
   const bool cp2 = col_scale & SMOE_COLSCALE_POW2, rp2 = col_scale & SMOE_ROWSCALE_POW2;
@@ -684,7 +691,11 @@ void combine_bwd_cols_launch(const uint16_t* dout, const int32_t* row_map, const
 }
 }  // namespace
 
-int smoe::combine_bwd_quant(const uint16_t* dout, const uint16_t* y, const int32_t* inv_map, const int32_t* row_map, const float* w, int T, int K, int H, const int32_t* offsets, int E, int ld, uint8_t* dyq, float* dys, uint8_t* dyTq, float* dyTs, int32_t* pad, bool make_pad, float* dw, int col_scale, void* stream) {
+int smoe::combine_bwd_quant(const uint16_t* dout, const uint16_t* y, const int32_t* inv_map,
+                            const int32_t* row_map, const float* w, int T, int K, int H,
+                            const int32_t* offsets, int E, int ld, uint8_t* dyq, float* dys,
+                            uint8_t* dyTq, float* dyTs, int32_t* pad, bool make_pad, float* dw,
+                            int col_scale, void* stream) {
   if (T <= 0 || H <= 0) return SMOE_EINVAL_DIM;
   if (col_scale & ~(SMOE_COLSCALE_POW2 | SMOE_ROWSCALE_POW2)) return SMOE_EINVAL_MODE;
   const bool cp2 = col_scale & SMOE_COLSCALE_POW2, rp2 = col_scale & SMOE_ROWSCALE_POW2;
@@ -728,7 +739,10 @@ int smoe::combine_bwd_quant(const uint16_t* dout, const uint16_t* y, const int32
   SMOE_RETURN_LAUNCH();
 }
 
-int smoe::combine_bwd_quant_cols(const uint16_t* dout, const int32_t* row_map, const float* w, int T, int K, int H, const int32_t* offsets, int E, int ld, uint8_t* dyTq, float* dyTs, int32_t* pad, bool make_pad, int col_scale, void* stream) {
+int smoe::combine_bwd_quant_cols(const uint16_t* dout, const int32_t* row_map, const float* w,
+                                 int T, int K, int H, const int32_t* offsets, int E, int ld,
+                                 uint8_t* dyTq, float* dyTs, int32_t* pad, bool make_pad,
+                                 int col_scale, void* stream) {
   if (T <= 0 || H <= 0) return SMOE_EINVAL_DIM;
   if (col_scale & ~SMOE_COLSCALE_POW2) return SMOE_EINVAL_MODE;
   if (H % kLane) return SMOE_EINVAL_ALIGN128;
@@ -752,9 +766,10 @@ int smoe::combine_bwd_quant_cols(const uint16_t* dout, const int32_t* row_map, c
 }
 
 // ------------------------------------------- the entry points of these
-extern "C" int smoe_quant_cols_128x1(const uint16_t* x, const int32_t* gather, int gather_div, int
-                                     R, int C, const int32_t* offsets, int E, int ld, uint8_t* xTq,
-                                     float* xTs, int32_t* pad, int col_scale, void* stream) {
+extern "C" int smoe_quant_cols_128x1(const uint16_t* x, const int32_t* gather, int gather_div,
+                                     int R, int C, const int32_t* offsets, int E, int ld,
+                                     uint8_t* xTq, float* xTs, int32_t* pad, int col_scale,
+                                     void* stream) {
   return quant_cols_128x1(x, gather, gather_div, R, C, offsets, E, ld, xTq, xTs, pad, true,
       col_scale, stream);
 }
@@ -765,28 +780,29 @@ extern "C" int smoe_quant_rows_cols(const uint16_t* x, int R, int C, const int32
   return quant_rows_cols(x, R, C, offsets, E, ld, xq, xs, xTq, xTs, pad, true, col_scale, stream);
 }
 
-extern "C" int smoe_swiglu_bwd_quant(const uint16_t* c1, const uint16_t* dh, int R, int I, const
-                                     int32_t* offsets, int E, int ld, uint8_t* dcq, float* dcs,
-                                     uint8_t* dcTq, float* dcTs, int32_t* pad, uint16_t* dc1, int
-                                     col_scale, void* stream) {
+extern "C" int smoe_swiglu_bwd_quant(const uint16_t* c1, const uint16_t* dh, int R, int I,
+                                     const int32_t* offsets, int E, int ld, uint8_t* dcq,
+                                     float* dcs, uint8_t* dcTq, float* dcTs, int32_t* pad,
+                                     uint16_t* dc1, int col_scale, void* stream) {
   return swiglu_bwd_quant(c1, dh, R, I, offsets, E, ld, dcq, dcs, dcTq, dcTs, pad, true, dc1,
       col_scale, stream);
 }
 
-extern "C" int smoe_unpermute_combine_bwd_quant(const uint16_t* dout, const uint16_t* y, const
-                                                int32_t* inv_map, const int32_t* row_map, const
-                                                float* w, int T, int K, int H, const int32_t*
-                                                offsets, int E, int ld, uint8_t* dyq, float* dys,
-                                                uint8_t* dyTq, float* dyTs, int32_t* pad, float* dw,
-                                                int col_scale, void* stream) {
+extern "C" int smoe_unpermute_combine_bwd_quant(const uint16_t* dout, const uint16_t* y,
+                                                const int32_t* inv_map, const int32_t* row_map,
+                                                const float* w, int T, int K, int H,
+                                                const int32_t* offsets, int E, int ld, uint8_t* dyq,
+                                                float* dys, uint8_t* dyTq, float* dyTs,
+                                                int32_t* pad, float* dw, int col_scale,
+                                                void* stream) {
   return combine_bwd_quant(dout, y, inv_map, row_map, w, T, K, H, offsets, E, ld, dyq, dys, dyTq,
       dyTs, pad, true, dw, col_scale, stream);
 }
 
-extern "C" int smoe_combine_bwd_quant_cols(const uint16_t* dout, const int32_t* row_map, const
-                                           float* w, int T, int K, int H, const int32_t* offsets,
-                                           int E, int ld, uint8_t* dyTq, float* dyTs, int32_t* pad,
-                                           int col_scale, void* stream) {
+extern "C" int smoe_combine_bwd_quant_cols(const uint16_t* dout, const int32_t* row_map,
+                                           const float* w, int T, int K, int H,
+                                           const int32_t* offsets, int E, int ld, uint8_t* dyTq,
+                                           float* dyTs, int32_t* pad, int col_scale, void* stream) {
   return combine_bwd_quant_cols(dout, row_map, w, T, K, H, offsets, E, ld, dyTq, dyTs, pad, true,
       col_scale, stream);
 }
