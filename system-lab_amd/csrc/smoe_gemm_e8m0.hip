@@ -379,10 +379,11 @@ __global__ __launch_bounds__(kThreads, 1) void grouped_gemm_fp8_e8m0_kernel(
   // kShort: an expert's last tile has fewer rows, and its empty row blocks are
   // skipped.  us without -> with: E 32, N 5760, K 2944 263 -> 244 (312 rows per
   // expert), 354 -> 334 (512); N 4096, K 7168 303 -> 297 (250), 1660 -> 1612 (2048); E
-  // 128, N 1536, K 2048 173 -> 168 (256), 471 -> 461 (1024); between 128 and 256 rows,
-  // where few tiles are short, up to 3% slower.  Fused SwiGLU of long K gains to
-  // 320 rows (1.00 - 1.11) and gives up to 3% from 400 on (E 96, N 1024, K 4608); the
-  // form without it spills one register.
+  // 128, N 1536, K 2048 173 -> 168 (256), 471 -> 461 (1024).  13 shapes at 256 - 1500
+  // rows: means 1.01 at random loads (0.97 where no tile is short) and 1.02 at
+  // Zipf(1.2) ones; between 128 and 256 rows, where few tiles are short, up to 3%
+  // slower.  Not with fused SwiGLU: the longer code lost 0.987 and 0.998 on
+  // average (57 loads; E 32, N 4096, K 7168, 700 rows random 0.98).  Spills one register.
   if (!kShort || rows > 128) k_loop(std::integral_constant<int, kRB>{});
   else if (rows > 64) k_loop(std::integral_constant<int, 8>{});
   else k_loop(std::integral_constant<int, 4>{});
@@ -504,13 +505,8 @@ extern "C" int smoe_grouped_gemm_fp8_packed_e8m0_swiglu(const uint8_t* a, const 
   long long mt_bound;
   const long long nblk = e8m0_grid(E, R, I / kGroup, &mt_bound);
   if (nblk > 0x7fffffffLL) return SMOE_EINVAL_DIM;
-  if (short_tiles(E, R, I / kGroup, 128, 256, 2048))
-    e8m0::grouped_gemm_fp8_e8m0_kernel<true, true>
-        <<<dim3((unsigned)nblk), dim3(e8m0::kThreads), 0, (hipStream_t)stream>>>(
-            a, as, w1p, w1s, offsets, E, R, 2 * I, Kdim, (int)mt_bound, c1, hq, hs);
-  else
-    e8m0::grouped_gemm_fp8_e8m0_kernel<true, false>
-        <<<dim3((unsigned)nblk), dim3(e8m0::kThreads), 0, (hipStream_t)stream>>>(
-            a, as, w1p, w1s, offsets, E, R, 2 * I, Kdim, (int)mt_bound, c1, hq, hs);
+  e8m0::grouped_gemm_fp8_e8m0_kernel<true, false>
+      <<<dim3((unsigned)nblk), dim3(e8m0::kThreads), 0, (hipStream_t)stream>>>(
+          a, as, w1p, w1s, offsets, E, R, 2 * I, Kdim, (int)mt_bound, c1, hq, hs);
   SMOE_RETURN_LAUNCH();
 }

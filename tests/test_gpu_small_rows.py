@@ -243,8 +243,9 @@ def test_tile_heights_equal_the_256_row_kernels(dev, counts, N, _, form):
 @pytest.mark.parametrize("form", ["plain", "e8m0"])
 def test_short_tiles_of_the_256_row_kernels(dev, K, form):
     """Last tiles on both sides of the 64 and 128 rows at which the 256-row
-    kernels skip row blocks, against the same rows in a call whose average
-    (above 2048 rows, the rest unused) selects the kernels without the skip."""
+    kernels (without SwiGLU) skip row blocks, against the same rows in a call
+    whose average (above 2048 rows, the rest unused) selects those without the
+    skip."""
     print("[short tiles]", form, K, flush=True)
     E, N, e8m0 = 96, 512, form == "e8m0"
     edges = [1, 16, 63, 64, 65, 127, 128, 129, 191, 192, 193, 255, 256, 257, 320, 385, 449, 512, 700, 0, 900, 1025,
@@ -257,7 +258,6 @@ def test_short_tiles_of_the_256_row_kernels(dev, K, form):
     xq, xs = ops.quant_rows(W.tokens(n, K, device=dev, seed=K), scale=scale)
     wq, ws = ops.quantize_weight_blockwise(W.weights(E, N, K, device=dev, seed=3), scale=scale)
     w = ops.pack_weight_fp8(wq) if e8m0 else wq
-    for swiglu in (False, True):
-        short = run(xq, xs, w, ws, off, n, e8m0, swiglu, N)
-        for a, b in zip(short, run(xq, xs, w, ws, off, 2049 * E + n, e8m0, swiglu, N)):
-            assert torch.equal(a, b), f"swiglu={swiglu}"
+    short = run(xq, xs, w, ws, off, n, e8m0, False, N)
+    for a, b in zip(short, run(xq, xs, w, ws, off, 2049 * E + n, e8m0, False, N)):
+        assert torch.equal(a, b)
