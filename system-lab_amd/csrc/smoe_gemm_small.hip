@@ -418,8 +418,9 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_small_kernel(
 //     E8M0 112 rows 132 -> 141, 75 rows and Zipf loads 158 -> 181
 //   plain, whose fragment loads touch 16 lines each: 65 rows (N 4096, K 7168) 246 ->
 //     199, 97 rows (N 5760, K 2944) 130 -> 152, 100 rows (N 4096, K 7168) 249 -> 289
-// Zipf(1.2) loads below the line gain as much or more (packed 100 rows, N 4096,
-// K 7168: 291 -> 227; plain 75 rows 259 -> 259).
+// Zipf(1.2) loads gain less near the line, where their tall experts' tiles make
+// a second, nearly empty round of workgroups: 0.91 - 1.2 of random ones (packed
+// 100 rows, N 4096, K 7168: 291 -> 227).  Not so well with plain weights: see 5.
 //
 // 2. A chip that 256 x 256 tiles leave mostly idle, any rows per expert: up to 96
 // such tiles this kernel's more and smaller ones gain 1.04 - 2.7 (E 8, N 1024, 512
@@ -448,6 +449,18 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_small_kernel(
 //   packed, K > 3072: 64 rows 1.12 (0.92) / 1.13 (0.95), 1.22 (0.98) / 1.16 (0.95); 72 rows
 //     0.96 (0.88) with SwiGLU; E8M0 64 rows 1.11 (0.95) / 1.11 (0.96), 72 rows 0.98 (0.95)
 //     with SwiGLU.  K <= 3072: as in 1.
+//
+// 5. Between one and a half and two rounds (384 < E * N/256 <= 512): experts with a
+// second tile push the launch past two workgroups per CU, and the few that are
+// over run alone.  Means and the worst, with SwiGLU / without, random then
+// Zipf(1.2) loads:
+//   plain, K > 2048 (13 shapes, E 8 - 96, K 3072 - 14336): 40 rows 1.28 (1.20) / 1.25
+//     (1.11), 1.20 (0.99) / 1.09 (0.95); 44 rows 1.26 (1.19) / 1.18 (1.07), 1.05 (0.89) / 1.02
+//     (0.84); 48 - 80 rows 1.16 (1.03) / 1.08 (0.87), 0.99 (0.84) / 0.95 (0.79)
+//   plain, K 2048, 48 - 80 rows: 1.40 (1.31) / 1.35 (1.18), 1.11 (0.91) / 1.04 (0.92)
+//   the packed forms stream faster and keep 1's lines: E8M0 48 - 80 rows 1.32 (1.16) /
+//     1.24 (0.96), 1.21 (0.91) / 1.11 (0.89); packed 48 - 88 rows 1.38 (1.22) / 1.31 (1.01),
+//     1.20 (0.96) / 1.15 (0.93), 96 - 112 rows 1.09 (0.90) / 1.06 (0.87), 1.28 (1.01) / 1.23 (0.96)
 bool small_gemm_rows(SmallWeights lay, bool e8m0, bool swiglu, int E, int R, int N, int Kdim) {
   const bool packed = lay == SmallWeights::kPacked;
   long long one_tile = !packed ? 80
@@ -458,6 +471,7 @@ bool small_gemm_rows(SmallWeights lay, bool e8m0, bool swiglu, int E, int R, int
     if (!packed) one_tile = t256 <= 192 ? 56 : 48;
     else if (Kdim > 3072) one_tile = 64;
   }
+  if (!packed && t256 > 384 && t256 <= 512 && Kdim > 2048) one_tile = 40;
   auto to = [&](long long rows) { return R <= rows * E; };
   if (to(one_tile)) return true;
   if ((packed || !swiglu) && (2LL * R + 256LL * E) * ((N + 255) / 256) <= 96 * 512) return true;
