@@ -73,7 +73,11 @@ struct WRing {
 // expert: bf16 704 -> 653, added into 1064 -> 748 (the old values are read
 // while the pass is staged), fp32 777 -> 769, added into 1183 -> 950; E8M0 642 ->
 // 609, 995 -> 680, 711 -> 723, 1129 -> 911.  E 32, N = K = 2880, 512 rows: bf16
-// 341 -> 305, fp32 341 -> 341.  Loading the next tile during the last step
+// 341 -> 305, fp32 341 -> 341.  fp32 without addition breaks even, as its four
+// passes cost what the early loads save: 9 shapes, random loads of 16 rows per expert
+// 0.97, 130 1.05, 512 1.02, 1024 0.99, Zipf(1.2) 0.97 - 1.00, a lone tile 0.9.  Two
+// passes of 128 rows for it, in all tiles or in those of more than 6 or 9 steps,
+// came to 0.97 - 1.00 (1.06 at 130 rows).  Loading the next tile during the last step
 // instead spilled (the loop body is at the register limit).
 template <int kOut, bool kE8M0>
 __device__ __forceinline__ void wgrad_tile(const uint8_t* __restrict__ aT,
