@@ -38,8 +38,8 @@ def _install_optimizer_hook():
 
 def _weight_is(w, s, E: int, N: int, Kd: int) -> bool:
     """w, s are an fp8 weight [E, N, K] (plain or packed) and its block scales."""
-    return (tuple(w.shape) == (E, N, ops.pad128(Kd))
-            and tuple(s.shape) == (E, ops.nblocks(N), ops.nblocks(Kd)))
+    kb = ops.nblocks(Kd)  # (torch.Size compares as a tuple: 2 us a forward less than conversions)
+    return w.shape == (E, N, kb * ops.GROUP) and s.shape == (E, ops.nblocks(N), kb)
 
 
 class _SimpleMoEFunction(torch.autograd.Function):
@@ -318,7 +318,10 @@ class SimpleMoE(nn.Module):
         gate = logits if logits is not None else self.w_gate.detach()
         ops._check(gate, "logits", (torch.float32,), 2)
         bias = self.router_bias
-        E, I = w1.shape[0], w1.shape[1] // 2
+        flags = self._layer_flags(w1, w2)
+        w1, w2 = ops._gemm_tensor(w1), ops._gemm_tensor(w2)
+        E, I, _ = w1.shape
+        I //= 2
         if bias is not None:
             ops._check(bias, "router_bias", (torch.float32,), 1)
             if bias.numel() != E:
@@ -327,16 +330,15 @@ class SimpleMoE(nn.Module):
             raise ValueError(f"the weights are on {w1.device} and {w2.device}, x on {dev}")
         # the native call takes the sizes as numbers: the tensors' own (weights
         # may be replaced by others), and only where every shape agrees
-        if not (tuple(gate.shape) == ((T if logits is not None else H), E)
+        if not (gate.shape == ((T if logits is not None else H), E)
                 and _weight_is(w1, w1s, E, 2 * I, H) and _weight_is(w2, w2s, E, H, I)):
             return self._forward_by_operators(x, logits, save)
-        flags = self._layer_flags(w1, w2)
         lib = _C.lib()
         out = torch.empty((T, H), dtype=torch.bfloat16, device=dev)
         ws = ops._status_workspace(lib.smoe_route_dispatch_workspace_size(T, H, E, K), dev)
         a = _C.LayerFwd(T, H, I, E, K, flags, x.data_ptr(), None if logits is None else gate.data_ptr(),
                         gate.data_ptr() if logits is None else None, None if bias is None else bias.data_ptr(),
-                        ops._gemm_ptr(w1), w1s.data_ptr(), ops._gemm_ptr(w2), w2s.data_ptr(), out.data_ptr(),
+                        w1.data_ptr(), w1s.data_ptr(), w2.data_ptr(), w2s.data_ptr(), out.data_ptr(),
                         ws.data_ptr(), ws.numel())
         inter = None
         if save:
@@ -517,7 +519,8 @@ class SimpleMoE(nn.Module):
         a = _C.LayerBwd(T, H, I, E, K, flags, modes[0], modes[1], dout.data_ptr(),
                         *(inter[k].data_ptr() for k in ("x", "logits", "topk_idx", "topk_w", "row_map",
                                                         "inv_map", "offsets", "c1", "h", "y")),
-                        ops._gemm_ptr(w1t), w1ts.data_ptr(), ops._gemm_ptr(w2t), w2ts.data_ptr(),
+                        ops._gemm_tensor(w1t).data_ptr(), w1ts.data_ptr(), ops._gemm_tensor(w2t).data_ptr(),
+                        w2ts.data_ptr(),
                         *(out[k].data_ptr() for k in ("dx", "dw1", "dw2", "dtopk_w", "dlogits", "dyq", "dys",
                                                       "dh", "dxs")),
                         scratch.data_ptr(), nbytes)

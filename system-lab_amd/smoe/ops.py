@@ -430,9 +430,9 @@ def quantize_pack_weight(w: torch.Tensor, scale: str = "amax"):
     return wq, ws, PackedWeight(wp)
 
 
-def _gemm_ptr(w) -> int:
-    """Address of a weight in the form the GEMMs take it."""
-    return (w.data if isinstance(w, PackedWeight) else w).data_ptr()
+def _gemm_tensor(w) -> torch.Tensor:
+    """The memory of a weight in the form the GEMMs take it."""
+    return w.data if isinstance(w, PackedWeight) else w
 
 
 def _weight(wq, name):
