@@ -220,9 +220,8 @@ def test_small_rows_equal_the_256_row_kernels(dev, counts, N, K, form):
 
 
 CUT_K = 1536
-# (above the line plain weights stay on the 256-row kernel)
-CUT_FORMS = [(f, c, N) for c, N, _ in CUT for f in ("plain", "packed", "e8m0")
-             if f != "plain" or small_cols(f, True, len(c), sum(c), N, CUT_K)]
+# (of these only the narrow loads are below the line of plain weights)
+CUT_FORMS = [(f, c, N) for c, N, _ in CUT for f in ("plain", "packed", "e8m0") if f != "plain" or N == 256]
 
 
 @pytest.mark.gpu

@@ -90,8 +90,9 @@ COLUMNS = [
     (TALL * 2, 2880, 128), ([65] * 16, 2576, 128),
     (TALL * 2, 272, 64), (TALL, 720, 64),
 ]
+# (65 rows are above the line of plain weights)
 COLUMNS = [(f, c, N, K, w) for c, N, w in COLUMNS for f, K in [("plain", 512), ("packed", 512), ("e8m0", 640)]
-           if small_cols(f, False, len(c), sum(c), N, K)]
+           if f != "plain" or N != 2576]
 
 
 def test_column_cases_cover_every_width_and_form():
